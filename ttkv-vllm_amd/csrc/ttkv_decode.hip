@@ -49,8 +49,17 @@
 #include <math.h>
 
 #include "ttkv_device.h"
+#include "ttkv_host.h"
 
 namespace ttkv {
+
+// the constant address space (kernel arguments, read with scalar loads); the host pass, which only
+// parses the kernels, does not know it
+#ifdef __HIP_DEVICE_COMPILE__
+#define AS4 __attribute__((address_space(4)))
+#else
+#define AS4
+#endif
 
 constexpr int kTile = 64;
 constexpr int kThreads = 256;
@@ -94,8 +103,22 @@ struct DecodeArgs {
   int chunk_cap, target, max_seq;  // chunk length cap, work items aimed at, longest context
 };
 
+// The kernels of one code width (the build compiles this file once per width, and once for the host
+// side): ku is the coefficient window in 16-wide k units.
+int decode_dispatch_3(const DecodeArgs& a, int ku, int grid, hipStream_t st);
+int decode_dispatch_4(const DecodeArgs& a, int ku, int grid, hipStream_t st);
+
+#ifdef TTKV_DECODE_BITS
+
 // KU = coefficient window in 16-wide k units: r1 is padded to 16 * KU; the reconstruction runs
 // KU / 2 MFMA steps of k = 32 and, for odd KU, one of k = 16.
+// One workgroup's segment: tiles [t0, t1) of request r, its chunk c of n_chunks, whose partials
+// start at `base`; and its team's units, for a range plan.
+struct Segment {
+  int32_t h, r, c, n_chunks, base, seq, qrow, dslot, t0, t1;
+  int32_t ranges, team, u_lo, u_hi, units, n_teams;
+};
+
 template <int KU, int G>
 struct DecodeSmem {
   static constexpr int kCoefStride = KU * 16 + 8;  // fp16 per token row
@@ -116,6 +139,12 @@ struct DecodeSmem {
   float f[2][kTile];   // cs * scale * log2(e), by tile parity
   float m[G], l[G];
   int is_last;
+  // the range plan's requests: first unit, length, decoder slot, query row
+  int32_t pl_start[kPlanReqs], pl_seq[kPlanReqs], pl_dec[kPlanReqs], pl_q[kPlanReqs];
+  // the segment in work and what is needed to open the next. Kept here and not in scalar registers,
+  // which the tile loop needs: with these values live across it the compiler gives up
+  // interleaving its MFMA and vector instructions (8 x 14,402: 133 against 126 us).
+  Segment sg;
 };
 
 // One-round split-K combine for up to NC chunks: each thread requests every chunk's (max, sum,
@@ -270,71 +299,323 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
   const int n_pairs = wave_sum_i(nreq_items);
   const int n_items = n_pairs * g.H;
   maxc = wave_max_i(maxc);
-  const int per_xcd = (n_items + 7) >> 3;
-  if ((int)(blockIdx.x >> 3) >= per_xcd) return;
-  const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (w >= n_items) return;
-  const int h = w % g.H;
-  const int j = w / g.H;
-  // (chunk c, request r) of pair j: c is the largest with P(c) <= j, P(c) = sum_r min(nch_r, c);
-  // r is the (j - P(c))-th request with more than c chunks; base = chunks of the requests before
-  // r (its partials follow theirs). When every request has the same count this is a division.
-  int c = 0, r = 0, base = 0;
-  if (n_pairs == maxc * a.num_reqs) {
-    c = j / a.num_reqs;
-    r = j - c * a.num_reqs;
-    base = r * maxc;
-  } else {
-    int pc = 0, hi = maxc;
-    while (hi - c > 1) {
-      const int mid = (c + hi) >> 1;
-      int pm = 0;
-#pragma unroll
-      for (int i = 0; i < kPlanLanes; ++i)
-        if (i < nper) pm += min(nchl[i], mid);
-      pm = wave_sum_i(pm);
-      if (pm <= j) {
-        c = mid;
-        pc = pm;
-      } else {
-        hi = mid;
-      }
-    }
-    int k = j - pc;
-    bool found = false;
+
+  // Where the chunks above leave the chip uneven -- requests of different lengths with only one or
+  // two chunks each, or a last round that is nearly empty -- the tiles of all requests are laid
+  // end to end instead and cut into equal ranges, one per team of H workgroups (one per head).
+  // A workgroup then walks its range request by request: the tail of one, whole ones, the head
+  // of another, each with its own decoder and its own partial. A request counts kOpen units more
+  // than its tiles, about what opening it costs. Ranges are taken where the chunk plan's longest
+  // workgroup has more than kUneven / 16 times a range's units, which batches of like lengths do
+  // not (8 x 14,402: 30 units against 30; 12 x 8,000, 1.07 times: 108 us in chunks, 110 in ranges).
+  // 61 requests of 70 .. 2,900 tokens (G = 4): one chunk per request, 46 tiles in the longest,
+  // 24 on average: 180 us; in ranges 110 us.
+  constexpr int kOpen = 1, kUneven = 18;
+  const int n_teams = max(1, a.target / g.H);
+  int units = 0;
+  bool ranges = false;
+  // (no batch of so few tokens takes ranges; one request never needs them)
+  if (a.num_reqs > 1 && tot / kTile + 2 * a.num_reqs > 2 * n_teams) {
+    int longest = 0;
 #pragma unroll
     for (int i = 0; i < kPlanLanes; ++i) {
-      if (i < nper && !found) {
-        const uint64_t msk = __builtin_amdgcn_ballot_w64(nchl[i] > c);
-        const int cnt = __builtin_popcountll(msk);
-        if (k < cnt) {
-          const uint64_t below = lane ? msk & (~0ull >> (64 - lane)) : 0ull;
-          const bool hit = ((msk >> lane) & 1ull) && __builtin_popcountll(below) == k;
-          r = 64 * i + __builtin_ctzll(__builtin_amdgcn_ballot_w64(hit));
-          found = true;
-        } else {
-          k -= cnt;
-        }
+      const int tiles = max(1, (seql[i] + kTile - 1) / kTile);
+      if (i < nper && lane + 64 * i < a.num_reqs) {
+        units += tiles + kOpen;
+        longest = max(longest, min(tiles, chunk / kTile));
       }
     }
-    int bl = 0;
-#pragma unroll
-    for (int i = 0; i < kPlanLanes; ++i)
-      if (i < nper) bl += lane + 64 * i < r ? nchl[i] : 0;
-    base = wave_sum_i(bl);
-  }
-  int n_chunks = 0, seq = 0, qrow_r = 0, dslot = -1;
-#pragma unroll
-  for (int i = 0; i < kPlanLanes; ++i) {
-    if ((r >> 6) == i) {
-      n_chunks = __builtin_amdgcn_readlane(nchl[i], r & 63);
-      seq = __builtin_amdgcn_readlane(seql[i], r & 63);
-      qrow_r = __builtin_amdgcn_readlane(qsll[i], r & 63);
-      dslot = __builtin_amdgcn_readlane(decl[i], r & 63);
-    }
+    units = wave_sum_i(units);
+    longest = wave_max_i(longest);
+    const int range_len = (units + n_teams - 1) / n_teams;
+    const int rounds_used = max(1, (n_items + a.target - 1) / a.target);
+    ranges = units > 2 * n_teams && range_len < a.chunk_cap / kTile &&
+             16 * rounds_used * (longest + kOpen) > kUneven * (range_len + kOpen);
   }
 
-  const int t0 = c * chunk;
+  const int n_work = ranges ? n_teams * g.H : n_items;
+  const int per_xcd = (n_work + 7) >> 3;
+  if ((int)(blockIdx.x >> 3) >= per_xcd) return;
+  const int w = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (w >= n_work) return;
+  const int h = w % g.H;
+  const int j = w / g.H;
+  int c = 0, r = 0, base = 0, n_chunks = 0, seq = 0, qrow_r = 0, dslot = -1, t0 = 0, t1 = 0;
+  int u_lo = 0, u_hi = 0;  // this team's units
+  // The segment of request r in the range of units [u_lo, u_hi) of team j; false when the range ends
+  // before the request's tiles.
+  auto open_range = [&](Segment& q) -> bool {
+    auto rfl = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    // the team that holds unit u
+    auto team_of = [&](int u) {
+      return (int)((((int64_t)u + 1) * q.n_teams + q.units - 1) / q.units) - 1;
+    };
+    const int start = rfl(S.pl_start[q.r]) + kOpen;  // unit of tile 0
+    q.seq = rfl(S.pl_seq[q.r]);
+    q.dslot = rfl(S.pl_dec[q.r]);
+    q.qrow = rfl(S.pl_q[q.r]);
+    const int tiles = max(1, (q.seq + kTile - 1) / kTile);
+    const int lo = max(q.u_lo, start), hi = min(q.u_hi, start + tiles);
+    if (lo >= hi) return false;
+    const int first = team_of(start);
+    q.n_chunks = team_of(start + tiles - 1) - first + 1;
+    q.c = q.team - first;
+    q.base = first + q.r;  // team + request rises with every segment: no two share a partial
+    q.t0 = (lo - start) * kTile;
+    q.t1 = min(q.seq, (hi - start) * kTile);
+    return true;
+  };
+  Segment q{};
+  if (ranges) {
+    // first units (a scan over the requests), staged with the rest of the plan
+    int before = 0;
+#pragma unroll
+    for (int i = 0; i < kPlanLanes; ++i) {
+      if (i < nper) {
+        const bool in = lane + 64 * i < a.num_reqs;
+        int v = in ? max(1, (seql[i] + kTile - 1) / kTile) + kOpen : 0;
+        const int own = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int up = __shfl_up(v, o);
+          v += lane >= o ? up : 0;
+        }
+        if (in && wv == 0) {
+          S.pl_start[lane + 64 * i] = before + v - own;
+          S.pl_seq[lane + 64 * i] = seql[i];
+          S.pl_dec[lane + 64 * i] = decl[i];
+          S.pl_q[lane + 64 * i] = qsll[i];
+        }
+        before += __builtin_amdgcn_readlane(v, 63);
+      }
+    }
+    u_lo = (int)((int64_t)units * j / n_teams);
+    u_hi = (int)((int64_t)units * (j + 1) / n_teams);
+    __syncthreads();
+    int below = 0;  // requests that start at or before u_lo
+#pragma unroll
+    for (int i = 0; i < kPlanLanes; ++i)
+      if (i < nper)
+        below += __builtin_popcountll(__builtin_amdgcn_ballot_w64(
+            lane + 64 * i < a.num_reqs && S.pl_start[min(lane + 64 * i, a.num_reqs - 1)] <= u_lo));
+    q = Segment{h, below - 1, 0, 0, 0, 0, 0, 0, 0, 0, 1, j, u_lo, u_hi, units, n_teams};
+    if (!open_range(q)) return;
+  } else {
+    // (chunk c, request r) of pair j: c is the largest with P(c) <= j, P(c) = sum_r min(nch_r, c);
+    // r is the (j - P(c))-th request with more than c chunks; base = chunks of the requests before
+    // r (its partials follow theirs). When every request has the same count this is a division.
+    if (n_pairs == maxc * a.num_reqs) {
+      c = j / a.num_reqs;
+      r = j - c * a.num_reqs;
+      base = r * maxc;
+    } else {
+      int pc = 0, hi = maxc;
+      while (hi - c > 1) {
+        const int mid = (c + hi) >> 1;
+        int pm = 0;
+#pragma unroll
+        for (int i = 0; i < kPlanLanes; ++i)
+          if (i < nper) pm += min(nchl[i], mid);
+        pm = wave_sum_i(pm);
+        if (pm <= j) {
+          c = mid;
+          pc = pm;
+        } else {
+          hi = mid;
+        }
+      }
+      int k = j - pc;
+      bool found = false;
+#pragma unroll
+      for (int i = 0; i < kPlanLanes; ++i) {
+        if (i < nper && !found) {
+          const uint64_t msk = __builtin_amdgcn_ballot_w64(nchl[i] > c);
+          const int cnt = __builtin_popcountll(msk);
+          if (k < cnt) {
+            const uint64_t below = lane ? msk & (~0ull >> (64 - lane)) : 0ull;
+            const bool hit = ((msk >> lane) & 1ull) && __builtin_popcountll(below) == k;
+            r = 64 * i + __builtin_ctzll(__builtin_amdgcn_ballot_w64(hit));
+            found = true;
+          } else {
+            k -= cnt;
+          }
+        }
+      }
+      int bl = 0;
+#pragma unroll
+      for (int i = 0; i < kPlanLanes; ++i)
+        if (i < nper) bl += lane + 64 * i < r ? nchl[i] : 0;
+      base = wave_sum_i(bl);
+    }
+#pragma unroll
+    for (int i = 0; i < kPlanLanes; ++i) {
+      if ((r >> 6) == i) {
+        n_chunks = __builtin_amdgcn_readlane(nchl[i], r & 63);
+        seq = __builtin_amdgcn_readlane(seql[i], r & 63);
+        qrow_r = __builtin_amdgcn_readlane(qsll[i], r & 63);
+        dslot = __builtin_amdgcn_readlane(decl[i], r & 63);
+      }
+    }
+    t0 = c * chunk;
+    t1 = min(seq, t0 + chunk);
+    q = Segment{h, r, c, n_chunks, base, seq, qrow_r, dslot, t0, t1, 0, 0, 0, 0, 0, 0};
+  }
+  // The end of a segment: its output, or its partial and, in the last workgroup of (request, head) to
+  // arrive, the combine.
+  auto finish = [&](const auto& a, int tid, float4v (&oacc)[2], float (&m_run)[G],
+                    float (&l_lane)[G], int ve) __attribute__((always_inline)) {
+  const Geom g = a.g;
+  const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
+  const int dl = 16 * wv + 4 * gq;
+  auto rfl = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int h = rfl(S.sg.h), r = rfl(S.sg.r), c = rfl(S.sg.c), n_chunks = rfl(S.sg.n_chunks),
+            base = rfl(S.sg.base);
+  const int64_t qrow = rfl(S.sg.qrow);
+  // the V-ruler scale 2^-ve taken back (exact)
+  if (ve != 0) {
+    const float vsc = ldexpf(1.f, ve);
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) oacc[mi] *= vsc;
+  }
+  // ---- normalisers: the per-lane partial sums over the wave (every wave holds the same)
+#pragma unroll
+  for (int p = 0; p < G; ++p) l_lane[p] = wave_sum(l_lane[p]);
+  if (tid == 0) {
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      S.m[p] = m_run[p];
+      S.l[p] = l_lane[p];
+    }
+  }
+  __syncthreads();
+
+  if (n_chunks == 1) {
+    if (n < G) {
+      const float inv = 1.f / S.l[n];
+      const int64_t ob = qrow * a.out_row_stride + (int64_t)(h * G + n) * kD;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        store_act(a.out, a.out_dtype, ob + dl + i, oacc[0][i] * inv);
+        store_act(a.out, a.out_dtype, ob + 64 + dl + i, oacc[1][i] * inv);
+      }
+    }
+    return;
+  }
+
+  // ---- split-K partial: [G][kD + 2] per (r, h, c): unnormalised o, running max, running sum
+  const int64_t pstride = (int64_t)G * (kD + 2);
+  float* partp = a.ws_part + ((int64_t)(base + c) * g.H + h) * pstride;
+  // The partial is written with agent-scope (write-through) atomic stores and waited on before
+  // the counter update, so no cache-wide release fence is needed.
+  auto st_agent = [](float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (n < G) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      st_agent(&partp[n * (kD + 2) + dl + i], oacc[0][i]);
+      st_agent(&partp[n * (kD + 2) + 64 + dl + i], oacc[1][i]);
+    }
+  }
+  if (tid < G) {
+    st_agent(&partp[tid * (kD + 2) + kD], S.m[tid]);
+    st_agent(&partp[tid * (kD + 2) + kD + 1], S.l[tid]);
+  }
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const int prev = arrive(&a.ws_cnt[r * g.H + h]);
+    S.is_last = (prev == n_chunks - 1);
+  }
+  __syncthreads();
+  if (!S.is_last) return;
+  // Every partial was stored write-through and completed before its counter update, so the
+  // agent-scope loads below (ld_agent: coherent across the XCDs' L2s, with no L2 invalidate) see
+  // them; the loads of all chunks are in flight together.
+
+  const float* pbase = a.ws_part + ((int64_t)base * g.H + h) * pstride;
+  const int64_t cstride = (int64_t)g.H * pstride;  // between chunks of one request and head
+  // Many chunks: weights in LDS (the tile buffers are free now) -- every chunk's (max, sum) in
+  // one round of loads, the per-head max and normaliser by one wave per head, then each output's
+  // chunk loads issued together: a few memory round trips whatever the chunk count. Up to 8
+  // chunks (24 for G <= 4), every value a thread's outputs need is requested in one round and
+  // combined in registers (combine_regs): one round trip. (Partials live past this XCD's L2; a round trip took ~2.8 us at
+  // the headline, and the former two rounds per output, four per thread, made this combine
+  // ~11.5 us of the launch's tail.)
+  float* wsh = reinterpret_cast<float*>(&S.coef[0][0]);
+  constexpr int kWCap = (int)(sizeof(S.coef) / sizeof(float));
+  const int ncp = n_chunks * G;
+  const int64_t orow = qrow * a.out_row_stride;
+  if (n_chunks <= 8) {
+    combine_regs<G, 8>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
+  } else if (G <= 4 && n_chunks <= 24) {
+    // (batch 1 at ~1k tokens: 17 chunks per head)
+    if constexpr (G <= 4) combine_regs<G, 24>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
+  } else if (2 * ncp <= kWCap) {
+    for (int i = tid; i < ncp; i += kThreads) {
+      const int cc = i / G, p = i - cc * G;
+      const float* pc = pbase + cc * cstride + p * (kD + 2);
+      wsh[i] = ld_agent(&pc[kD]);
+      wsh[ncp + i] = ld_agent(&pc[kD + 1]);
+    }
+    __syncthreads();
+    for (int p = wv; p < G; p += kWaves) {  // wave-uniform: whole waves take a head each
+      float mx = -INFINITY;
+      for (int cc = lane; cc < n_chunks; cc += 64) mx = fmaxf(mx, wsh[cc * G + p]);
+      mx = wave_max(mx);
+      float L = 0.f;
+      for (int cc = lane; cc < n_chunks; cc += 64)
+        L = fmaf(wsh[ncp + cc * G + p], exp2f(wsh[cc * G + p] - mx), L);
+      const float invL = 1.f / wave_sum(L);
+      for (int cc = lane; cc < n_chunks; cc += 64)
+        wsh[cc * G + p] = exp2f(wsh[cc * G + p] - mx) * invL;
+    }
+    __syncthreads();
+    for (int it = tid; it < G * kD; it += kThreads) {
+      const int p = it / kD;
+      const int dim = it - p * kD;
+      const float* po = pbase + p * (kD + 2) + dim;
+      float O = 0.f;
+      for (int c0 = 0; c0 < n_chunks; c0 += 32) {
+        float v[32];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) v[j] = c0 + j < n_chunks ? ld_agent(&po[(c0 + j) * cstride]) : 0.f;
+#pragma unroll
+        for (int j = 0; j < 32; ++j)
+          if (c0 + j < n_chunks) O = fmaf(v[j], wsh[(c0 + j) * G + p], O);
+      }
+      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim, O);
+    }
+  } else {  // more chunks than the LDS weights hold: two passes per output
+    for (int it = tid; it < G * kD; it += kThreads) {
+      const int p = it / kD;
+      const int dim = it - p * kD;
+      float M = -INFINITY;
+#pragma unroll 8
+      for (int cc = 0; cc < n_chunks; ++cc) M = fmaxf(M, ld_agent(&pbase[cc * cstride + p * (kD + 2) + kD]));
+      float L = 0.f, O = 0.f;
+#pragma unroll 8
+      for (int cc = 0; cc < n_chunks; ++cc) {
+        const float* pc = pbase + cc * cstride + p * (kD + 2);
+        const float f = exp2f(ld_agent(&pc[kD]) - M);
+        L = fmaf(ld_agent(&pc[kD + 1]), f, L);
+        O = fmaf(ld_agent(&pc[dim]), f, O);
+      }
+      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim,
+                O / L);
+    }
+  }
+  if (tid == 0) __hip_atomic_store(&a.ws_cnt[r * g.H + h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+
+  // One segment: the tiles [t0, t1) of request r (its chunk c of n_chunks) for head h.
+  auto segment = [&](const Segment& q, bool& need_luts, const auto& a, int tid) __attribute__((always_inline)) {
+  // (a copy: through a generic reference its fields would be loaded from memory in every tile)
+  const Geom g = a.g;
+  const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
+  if (tid == 0) S.sg = q;  // read back behind the barriers below
+  const int h = q.h, r = q.r, c = q.c, seq = q.seq, qrow_r = q.qrow, dslot = q.dslot, t0 = q.t0,
+            t1 = q.t1;
   const int ptok = tid >> 2;  // token / part handled by this thread in prefetch + commit
   const int part = tid & 3;
   // block id of this thread's token in the first tile (position clamped into the context)
@@ -348,8 +629,6 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
       store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G) * kD + i, 0.f);
     return;
   }
-  const int t1 = min(seq, t0 + chunk);
-
   // This chunk's block ids (at most kSegMax, host-bounded), requested in the same round trip as
   // the first tile's block id and the decoder slot: they depend on the plan only, and are staged
   // into LDS after the code tables are built.
@@ -426,7 +705,8 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
   }
 
   // ---- code tables, and this chunk's block ids
-  build_luts(S.lut, (RB == 3 || VB == 3) ? lut3s : nullptr, tid, kThreads);
+  if (need_luts) build_luts(S.lut, (RB == 3 || VB == 3) ? lut3s : nullptr, tid, kThreads);
+  need_luts = false;  // (a segment without tokens or decoder returns before this)
 #pragma unroll
   for (int k = 0; k < kSegPer; ++k) {
     const int i = tid + kThreads * k;
@@ -773,148 +1053,36 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
     }
   }
 
-  // the V-ruler scale 2^-ve taken back (exact)
-  if (ve != 0) {
-    const float vsc = ldexpf(1.f, ve);
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi) oacc[mi] *= vsc;
-  }
-  // ---- normalisers: the per-lane partial sums over the wave (every wave holds the same)
-#pragma unroll
-  for (int p = 0; p < G; ++p) l_lane[p] = wave_sum(l_lane[p]);
-  if (tid == 0) {
-#pragma unroll
-    for (int p = 0; p < G; ++p) {
-      S.m[p] = m_run[p];
-      S.l[p] = l_lane[p];
-    }
-  }
-  __syncthreads();
-
-  if (n_chunks == 1) {
-    if (n < G) {
-      const float inv = 1.f / S.l[n];
-      const int64_t ob = qrow * a.out_row_stride + (int64_t)(h * G + n) * kD;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        store_act(a.out, a.out_dtype, ob + dl + i, oacc[0][i] * inv);
-        store_act(a.out, a.out_dtype, ob + 64 + dl + i, oacc[1][i] * inv);
-      }
-    }
-    return;
-  }
-
-  // ---- split-K partial: [G][kD + 2] per (r, h, c): unnormalised o, running max, running sum
-  const int64_t pstride = (int64_t)G * (kD + 2);
-  float* partp = a.ws_part + ((int64_t)(base + c) * g.H + h) * pstride;
-  // The partial is written with agent-scope (write-through) atomic stores and waited on before
-  // the counter update, so no cache-wide release fence is needed.
-  auto st_agent = [](float* p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // What the rest needs of the segment and of the arguments is read again here, so that it does not
+  // take registers through the tile loop.
+  const DecodeArgs AS4* ap2 = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(ap2));
+  finish(*ap2, tid, oacc, m_run, l_lane, ve);
   };
-  if (n < G) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      st_agent(&partp[n * (kD + 2) + dl + i], oacc[0][i]);
-      st_agent(&partp[n * (kD + 2) + 64 + dl + i], oacc[1][i]);
-    }
-  }
-  if (tid < G) {
-    st_agent(&partp[tid * (kD + 2) + kD], S.m[tid]);
-    st_agent(&partp[tid * (kD + 2) + kD + 1], S.l[tid]);
-  }
-  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    const int prev = arrive(&a.ws_cnt[r * g.H + h]);
-    S.is_last = (prev == n_chunks - 1);
-  }
-  __syncthreads();
-  if (!S.is_last) return;
-  // Every partial was stored write-through and completed before its counter update, so the
-  // agent-scope loads below (ld_agent: coherent across the XCDs' L2s, with no L2 invalidate) see
-  // them; the loads of all chunks are in flight together.
 
-  const float* pbase = a.ws_part + ((int64_t)base * g.H + h) * pstride;
-  const int64_t cstride = (int64_t)g.H * pstride;  // between chunks of one request and head
-  // Many chunks: weights in LDS (the tile buffers are free now) -- every chunk's (max, sum) in
-  // one round of loads, the per-head max and normaliser by one wave per head, then each output's
-  // chunk loads issued together: a few memory round trips whatever the chunk count. Up to 8
-  // chunks (24 for G <= 4), every value a thread's outputs need is requested in one round and
-  // combined in registers (combine_regs): one round trip. (Partials live past this XCD's L2; a round trip took ~2.8 us at
-  // the headline, and the former two rounds per output, four per thread, made this combine
-  // ~11.5 us of the launch's tail.)
-  float* wsh = reinterpret_cast<float*>(&S.coef[0][0]);
-  constexpr int kWCap = (int)(sizeof(S.coef) / sizeof(float));
-  const int ncp = n_chunks * G;
-  const int64_t orow = qrow * a.out_row_stride;
-  if (n_chunks <= 8) {
-    combine_regs<G, 8>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
-  } else if (G <= 4 && n_chunks <= 24) {
-    // (batch 1 at ~1k tokens: 17 chunks per head)
-    if constexpr (G <= 4) combine_regs<G, 24>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
-  } else if (2 * ncp <= kWCap) {
-    for (int i = tid; i < ncp; i += kThreads) {
-      const int cc = i / G, p = i - cc * G;
-      const float* pc = pbase + cc * cstride + p * (kD + 2);
-      wsh[i] = ld_agent(&pc[kD]);
-      wsh[ncp + i] = ld_agent(&pc[kD + 1]);
-    }
-    __syncthreads();
-    for (int p = wv; p < G; p += kWaves) {  // wave-uniform: whole waves take a head each
-      float mx = -INFINITY;
-      for (int cc = lane; cc < n_chunks; cc += 64) mx = fmaxf(mx, wsh[cc * G + p]);
-      mx = wave_max(mx);
-      float L = 0.f;
-      for (int cc = lane; cc < n_chunks; cc += 64)
-        L = fmaf(wsh[ncp + cc * G + p], exp2f(wsh[cc * G + p] - mx), L);
-      const float invL = 1.f / wave_sum(L);
-      for (int cc = lane; cc < n_chunks; cc += 64)
-        wsh[cc * G + p] = exp2f(wsh[cc * G + p] - mx) * invL;
-    }
-    __syncthreads();
-    for (int it = tid; it < G * kD; it += kThreads) {
-      const int p = it / kD;
-      const int dim = it - p * kD;
-      const float* po = pbase + p * (kD + 2) + dim;
-      float O = 0.f;
-      for (int c0 = 0; c0 < n_chunks; c0 += 32) {
-        float v[32];
+
+  for (bool need_luts = true;;) {
+    // The arguments and the thread id go through opaque copies, so that what a segment derives from
+    // them is computed again for each: hoisted out of this loop it would not fit the registers.
+    const DecodeArgs AS4* ap = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();
+    int t = tid;
+    __asm__ volatile("" : "+s"(ap), "+v"(t));
+    segment(q, need_luts, *ap, t);
+    __syncthreads();  // every wave is done with the segment and its LDS
+    {
+      const int32_t* src = &S.sg.h;
+      int32_t* dst = &q.h;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = c0 + j < n_chunks ? ld_agent(&po[(c0 + j) * cstride]) : 0.f;
-#pragma unroll
-        for (int j = 0; j < 32; ++j)
-          if (c0 + j < n_chunks) O = fmaf(v[j], wsh[(c0 + j) * G + p], O);
-      }
-      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim, O);
+      for (int i = 0; i < (int)(sizeof(Segment) / 4); ++i)
+        dst[i] = __builtin_amdgcn_readfirstlane(src[i]);
     }
-  } else {  // more chunks than the LDS weights hold: two passes per output
-    for (int it = tid; it < G * kD; it += kThreads) {
-      const int p = it / kD;
-      const int dim = it - p * kD;
-      float M = -INFINITY;
-#pragma unroll 8
-      for (int cc = 0; cc < n_chunks; ++cc) M = fmaxf(M, ld_agent(&pbase[cc * cstride + p * (kD + 2) + kD]));
-      float L = 0.f, O = 0.f;
-#pragma unroll 8
-      for (int cc = 0; cc < n_chunks; ++cc) {
-        const float* pc = pbase + cc * cstride + p * (kD + 2);
-        const float f = exp2f(ld_agent(&pc[kD]) - M);
-        L = fmaf(ld_agent(&pc[kD + 1]), f, L);
-        O = fmaf(ld_agent(&pc[dim]), f, O);
-      }
-      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim,
-                O / L);
-    }
+    if (!q.ranges || ++q.r >= ap->num_reqs || !open_range(q)) return;
+    __syncthreads();  // every wave has read the last segment
   }
-  if (tid == 0) __hip_atomic_store(&a.ws_cnt[r * g.H + h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace ttkv
 
-
-// ------------------------------------------------------------------------------------ host side
-#include "ttkv_host.h"
 
 namespace ttkv {
 
@@ -966,6 +1134,20 @@ static int dispatch_k(const DecodeArgs& a, int ku, int grid, hipStream_t st) {
   }
   return host_fail(TTKV_E_UNSUPPORTED, "r1 > 160 is not built");
 }
+
+#if TTKV_DECODE_BITS == 3
+int decode_dispatch_3(const DecodeArgs& a, int ku, int grid, hipStream_t st) {
+  return dispatch_k<3, 3>(a, ku, grid, st);
+}
+#else
+int decode_dispatch_4(const DecodeArgs& a, int ku, int grid, hipStream_t st) {
+  return dispatch_k<4, 4>(a, ku, grid, st);
+}
+#endif
+
+}  // namespace ttkv
+
+#else  // the host side
 
 // Requests per launch: the work plan holds kPlanReqs of them, and a launch's token total must fit
 // an int. Larger batches run as several launches over consecutive request ranges.
@@ -1108,8 +1290,8 @@ int decode_paged(const Geom& g, int HQ, float scale, const void* q, int q_dtype,
       b.ws_part = (float*)((char*)ws + kCounterBytes);
     }
     const int grid = (int)((sh.items_cap + 7) / 8 * 8);
-    const int rc = g.res_bits == 3 ? dispatch_k<3, 3>(b, ku, grid, st)
-                                   : dispatch_k<4, 4>(b, ku, grid, st);
+    const int rc = g.res_bits == 3 ? decode_dispatch_3(b, ku, grid, st)
+                                   : decode_dispatch_4(b, ku, grid, st);
     if (rc != TTKV_OK) return rc;
   }
   return TTKV_OK;
@@ -1199,3 +1381,4 @@ int decode_paged_noalloc(const Geom& g, int HQ, float scale, const void* q, int 
 }
 
 }  // namespace ttkv
+#endif  // TTKV_DECODE_BITS
