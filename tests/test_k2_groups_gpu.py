@@ -1,0 +1,56 @@
+"""K2 attention at the edges of its work items: four query heads per KV head (24 groups of 16 rows
+over 8 waves), chunks of at most half an item's queries (the waves of a pair take half of every
+tile's keys each), and last blocks of one query, against the CPU oracle."""
+import pytest
+import torch
+
+from helpers import dec_pool_of, fitted_store, llama3_cache, paged
+from oracle import attend
+from vllm_ttkv import kernels, synth
+
+pytestmark = pytest.mark.gpu
+SCALE = 128 ** -0.5
+
+
+@pytest.mark.parametrize("cfg,H,G,r1,dtype,lens,qlens", [
+    ("safe", 8, 4, 110, torch.float16, [700, 333, 65], [49, 48, 64]),   # one past half, half
+    ("campaign4x", 8, 4, 110, torch.bfloat16, [900, 97], [97, 96]),     # one past an item
+    ("safe", 4, 4, 64, torch.float16, [1500], [2]),
+    ("tight", 8, 4, 128, torch.float16, [400, 401, 402], [17, 1, 200]),
+    ("safe", 8, 3, 110, torch.float16, [700, 640, 64], [65, 64, 16]),   # one past half, half
+    ("campaign4x", 8, 3, 96, torch.float16, [515, 130], [129, 19]),
+    ("safe", 8, 3, 110, torch.float16, [3000], [5]),                    # many key splits
+    ("safe", 8, 2, 110, torch.float16, [300, 200], [33, 128]),
+    ("safe", 2, 1, 110, torch.bfloat16, [300, 70], [64, 70]),           # a whole context
+])
+def test_row_groups(cfg, H, G, r1, dtype, lens, qlens):
+    print(f"[k2 groups] {cfg} H={H} G={G} r1={r1} {lens} {qlens}", flush=True)
+    stores = [fitted_store(cfg, n, seed=40 + i, r1=r1, H_=H) for i, n in enumerate(lens)]
+    pg = paged(stores, 16, 3)
+    lay = stores[0]["lay"]
+    q = synth.queries(sum(qlens), HQ=H * G, seed=9, dtype=dtype)
+    qsl = torch.tensor([0] + list(torch.tensor(qlens).cumsum(0)), dtype=torch.int32)
+    cache = llama3_cache(4096)
+    dev = "cuda"
+    dec_map = torch.full((pg["num_blocks"],), -1, dtype=torch.int32)
+    for r in range(len(lens)):
+        dec_map[pg["block_table"][r, 0]] = r
+    out = torch.full((sum(qlens), H * G, 128), float("nan"), dtype=dtype, device=dev)
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    ws = kernels.prefill_workspace(lay, H * G, len(lens), max(qlens), max(lens), dev)
+    args = (lay, q.to(dev), pg["page"].to(dev), 16, pg["block_table"].to(dev),
+            pg["seq_lens"].to(dev), qsl.to(dev), max(qlens), max(lens), dec_map.to(dev),
+            dec_pool_of([s["decoder"] for s in stores], dev), cache.to(dev), SCALE)
+    kernels.prefill_paged(*args, out=out, workspace=ws, error_word=err)
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    first = out.float().cpu()
+    kernels.prefill_paged(*args, out=out.fill_(0), workspace=ws, error_word=err)
+    assert torch.equal(out.float().cpu(), first)        # the counters came back to zero
+    want = attend.paged_continuation(lay, pg["page"], pg["block_table"], pg["seq_lens"], qsl,
+                                     q.float(), [s["decoder"] for s in stores], cache, 16, SCALE,
+                                     dtype=torch.float64)
+    tol = 1.0 if dtype == torch.float16 else 8.0        # bf16 rounds the output 8 times coarser
+    for r in range(len(lens)):
+        e = (first[qsl[r]:qsl[r + 1]].double() - want[r]).abs()
+        assert e.max() <= tol * 2e-3 and e.mean() <= tol * 1e-3, (r, e.max(), e.mean())

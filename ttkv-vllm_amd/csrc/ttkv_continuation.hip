@@ -43,7 +43,12 @@ namespace ttkv {
 constexpr int kXTile = 64;                 // keys per tile
 constexpr int kXThreads = 256;             // expand workgroup
 constexpr int kAThreads = 512;             // attend workgroup (8 waves)
-constexpr int kAQ = 128;                   // queries per attend work item (16 per wave)
+constexpr int kAQ = 128;                   // queries per work item (16 per wave and head), G <= 3
+// An attend wave holds up to three groups of 16 query rows (its registers' worth). With G <= 3
+// query heads per KV head it takes the G heads of 16 queries; with G = 4 the 8 waves take the 24
+// (head, 16 queries) groups of 96 queries, three each.
+__host__ __device__ constexpr int attend_groups(int G) { return G <= 3 ? G : 3; }
+__host__ __device__ constexpr int attend_queries(int G) { return G <= 3 ? kAQ : 96; }
 constexpr int kXSeg = 260;                 // block ids of one expand item staged in LDS
 constexpr int kTileKhi = 0;                // byte offsets inside one workspace tile
 constexpr int kTileKlo = kXTile * kD * 2;
@@ -390,14 +395,17 @@ struct AttendSmem {
   int is_last;
 };
 
-template <int G>
+template <int G, bool PAIR>
 __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
+  constexpr int NG = attend_groups(G);   // groups of 16 rows per wave
+  constexpr int AQ = attend_queries(G);  // queries per item
   extern __shared__ __align__(16) unsigned char smem_raw[];
   AttendSmem& S = *reinterpret_cast<AttendSmem*>(smem_raw);
   const Geom& g = a.g;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wv = tid >> 6;
+  // (scalar only for PAIR: as a scalar branch, the other kernel's two orders below spill)
+  const int wv = PAIR ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   const int n = lane & 15;
   const int gq = lane >> 4;
 
@@ -424,13 +432,13 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     qlen = min(qlen, a.max_q);
   }
   const int p0 = seq - qlen;
-  const int qa = qb * kAQ;
+  const int qa = qb * AQ;
   if (qlen <= 0 || qa >= qlen) return;
   if (p0 < 0) {
     if (lead) atomicOr(a.err, TTKV_ERR_SEQ_LEN);
     return;
   }
-  const int qe = min(qlen, qa + kAQ);
+  const int qe = min(qlen, qa + AQ);
   const int kmax = min(seq, p0 + qe);  // keys any query of the block may see
   const int nparts = (kmax + a.kchunk - 1) / a.kchunk;
   if (sp >= nparts) return;
@@ -485,30 +493,39 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
       __builtin_amdgcn_global_load_lds(gbl(src + 3072 + lane), (lds_ptr)((u32x4*)&T + 3072), 16, 0, 0);
   };
 
-  // query fragments (B operand of S^T = K Q^T): column n = query qa + 16 wv + n of head h*G+gg
-  const int qj = qa + 16 * wv + n;
-  const bool qvalid = qj < qe;
-  half8 qf[G][4];
+  // Row groups of this wave: group i is head hd(i), queries qa + 16 qg(i) + n. PAIR: chunks of at
+  // most AQ / 2 queries are laid out over four row waves, and waves 4 .. 7 take the second half of
+  // every tile's keys for the same rows. (A kernel of its own: with both layouts in one the long
+  // chunks ran 4 % slower.)
+  const int rw = PAIR ? wv & 3 : wv;
+  auto hd = [&](int i) { return G <= 3 ? i : (NG * rw + i) & 3; };
+  auto qg = [&](int i) { return G <= 3 ? rw : (NG * rw + i) >> 2; };
+  const bool active = qa + 16 * qg(0) < qe;  // (groups only rise within a wave)
+  // query fragments (B operand of S^T = K Q^T): column n = query n of the group
+  half8 qf[NG][4];
   {
     const bool qvec = act_rows_aligned(a.q, a.q_dtype, a.q_row_stride);
     // k-step ks, lane group gq: the dims of key chunk 4 ks + gq (tile_dims)
-    const int64_t qrow = (int64_t)(q0 + (qvalid ? qj : qa)) * a.q_row_stride + (int64_t)h * G * kD +
-                         4 * gq;
 #pragma unroll
-    for (int gg = 0; gg < G; ++gg)
+    for (int gg = 0; gg < NG; ++gg) {
+      const int qj = qa + 16 * qg(gg) + n;
+      const bool qvalid = qj < qe;
+      const int64_t qrow = (int64_t)(q0 + (qvalid ? qj : qa)) * a.q_row_stride +
+                           (int64_t)(h * G + hd(gg)) * kD + 4 * gq;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         float tq[8];
-        load_act_n<4>(a.q, a.q_dtype, qrow + (int64_t)gg * kD + 16 * ks, qvec, tq);
-        load_act_n<4>(a.q, a.q_dtype, qrow + (int64_t)gg * kD + 64 + 16 * ks, qvec, tq + 4);
+        load_act_n<4>(a.q, a.q_dtype, qrow + 16 * ks, qvec, tq);
+        load_act_n<4>(a.q, a.q_dtype, qrow + 64 + 16 * ks, qvec, tq + 4);
 #pragma unroll
         for (int i = 0; i < 8; ++i) qf[gg][ks][i] = qvalid ? (_Float16)tq[i] : (_Float16)0.0f;
       }
+    }
   }
-  float4v o[8][G];
-  float m_run[G], l_run[G];
+  float4v o[8][NG];
+  float m_run[NG], l_run[NG];
 #pragma unroll
-  for (int gg = 0; gg < G; ++gg) {
+  for (int gg = 0; gg < NG; ++gg) {
     m_run[gg] = -INFINITY;
     l_run[gg] = 0.f;
 #pragma unroll
@@ -516,7 +533,6 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
   }
 
   const int tl0 = k0 / kXTile, ntl_item = (k1 + kXTile - 1) / kXTile - tl0;
-  const int lim = p0 + qj;  // last key this lane's query may see
   const float sl2 = a.scale_log2;
 
   // One half step: keys 32 hf .. 32 hf + 31 of tile tl (buffer T): scores, softmax, P.V.
@@ -525,12 +541,10 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
   uint32_t koff[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) koff[ks] = n * 256 + (((4 * ks + gq) ^ (n & 7)) << 4);
-  uint32_t voff[2];
+  const uint32_t voff0 = 32768 + n * 128 + ((gq ^ (n & 7)) << 4);  // half 1: ^ 64
+  float l_lane[NG];  // per-lane partial normalisers, summed over the column at the end
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) voff[hf] = 32768 + n * 128 + (((4 * hf + gq) ^ (n & 7)) << 4);
-  float l_lane[G];  // per-lane partial normalisers, summed over the column at the end
-#pragma unroll
-  for (int gg = 0; gg < G; ++gg) l_lane[gg] = 0.f;
+  for (int gg = 0; gg < NG; ++gg) l_lane[gg] = 0.f;
   // P * ruler_v is carried at scale 2^-ve so that it stays an fp16 normal below 2^15 (P <= 2^8):
   // ve grows, behind a ballot, when a half step brings a ruler of 2^(7 + ve) or more, and the
   // wave's accumulators are rescaled by an exact power of two (ve is per wave: its own rows)
@@ -541,7 +555,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     const int tt = tl * kXTile;
     const char* tb = (const char*)&T;
     // -------------------------------------------------------- scores S^T = K Q^T
-    float4v sacc[2][G];
+    float4v sacc[2][NG];
 #pragma unroll
     for (int k2 = 0; k2 < 2; ++k2) {
       const char* rb = tb + (32 * hf + 16 * k2) * 256;
@@ -550,7 +564,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
         const half8 ka = *(const half8*)(rb + koff[ks]);
         const half8 kl = *(const half8*)(rb + 16384 + koff[ks]);
 #pragma unroll
-        for (int gg = 0; gg < G; ++gg) {
+        for (int gg = 0; gg < NG; ++gg) {
           sacc[k2][gg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
               ka, qf[gg][ks], ks ? sacc[k2][gg] : float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
           sacc[k2][gg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qf[gg][ks], sacc[k2][gg], 0, 0, 0);
@@ -561,14 +575,15 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     // key t is visible to this lane's query iff t <= min(k1 - 1, p0 + qj); a tile whose every
     // key is visible to the block's first query needs no mask (a uniform branch)
     if (!(tt + kXTile <= k1 && tt + kXTile - 1 <= p0 + qa)) {
-      const int last = min(k1 - 1, lim) - (tt + 32 * hf + 4 * gq);
 #pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2)
+      for (int gg = 0; gg < NG; ++gg) {
+        const int last = min(k1 - 1, p0 + qa + 16 * qg(gg) + n) - (tt + 32 * hf + 4 * gq);
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
+        for (int k2 = 0; k2 < 2; ++k2)
 #pragma unroll
-          for (int gg = 0; gg < G; ++gg)
+          for (int jj = 0; jj < 4; ++jj)
             sacc[k2][gg][jj] = 16 * k2 + jj <= last ? sacc[k2][gg][jj] : -INFINITY;
+      }
     }
     // -------------------------------------------------------- online softmax per column
     // (raw scores; the scale enters the exponent's fma, and m_run is in scaled units)
@@ -584,7 +599,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-          for (int gg = 0; gg < G; ++gg) o[dt][gg] *= f;
+          for (int gg = 0; gg < NG; ++gg) o[dt][gg] *= f;
         ve = ve_new;
         v_thr = ldexpf(1.f, 7 + ve);
         v_mul = ldexpf(1.f, -ve);
@@ -592,9 +607,9 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
       vr0 *= v_mul;
       vr1 *= v_mul;
     }
-    half8 pb[G];
+    half8 pb[NG];
 #pragma unroll
-    for (int gg = 0; gg < G; ++gg) {
+    for (int gg = 0; gg < NG; ++gg) {
       const float m01 = max3_mfma(sacc[0][gg][0], sacc[0][gg][1], sacc[0][gg][2]);
       const float m23 = max3_mfma(sacc[0][gg][3], sacc[1][gg][0], sacc[1][gg][1]);
       float mt = max3_mfma(m01, m23, max3_mfma(sacc[1][gg][2], sacc[1][gg][3], sacc[1][gg][3]));
@@ -626,9 +641,9 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     // -------------------------------------------------------- O^T += Vt (P ruler_v)^T
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
-      const half8 va = *(const half8*)(tb + dt * 2048 + voff[hf]);
+      const half8 va = *(const half8*)(tb + dt * 2048 + (voff0 ^ (hf << 6)));
 #pragma unroll
-      for (int gg = 0; gg < G; ++gg)
+      for (int gg = 0; gg < NG; ++gg)
         o[dt][gg] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb[gg], o[dt][gg], 0, 0, 0);
     }
   };
@@ -646,7 +661,10 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (k + 1 < ntl_item) dma_tile(S.t[(k + 1) % 3], tl0 + k + 1);
-    if (!late) {
+    if constexpr (PAIR) {
+      // (a wave without a query only moves its share of the tiles)
+      if (active && k < ntl_item) half_step(S.t[k % 3], tl0 + k, (int)late);
+    } else if (!late) {
       if (k < ntl_item) {
         half_step(S.t[k % 3], tl0 + k, 0);
         half_step(S.t[k % 3], tl0 + k, 1);
@@ -658,24 +676,63 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
   }
 
 #pragma unroll
-  for (int gg = 0; gg < G; ++gg) l_run[gg] = cross_row_sum(l_lane[gg]);
+  for (int gg = 0; gg < NG; ++gg) l_run[gg] = cross_row_sum(l_lane[gg]);
   if (ve != 0) {  // the V-ruler scale taken back (exact)
     const float vsc = ldexpf(1.f, ve);
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
-      for (int gg = 0; gg < G; ++gg) o[dt][gg] *= vsc;
+      for (int gg = 0; gg < NG; ++gg) o[dt][gg] *= vsc;
   }
+
+  // The two halves of a pair's keys: waves 4 .. 7 hand their (m, l, o) to waves 0 .. 3 through the
+  // tile buffers.
+  if constexpr (PAIR) {
+    constexpr int kRegs = NG * 34;  // floats per lane
+    float* mine = (float*)&S.t[0] + (int64_t)rw * kRegs * 64 + lane;
+    __syncthreads();
+    if (late) {
+#pragma unroll
+      for (int gg = 0; gg < NG; ++gg) {
+        mine[(34 * gg) * 64] = m_run[gg];
+        mine[(34 * gg + 1) * 64] = l_run[gg];
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mine[(34 * gg + 2 + 4 * dt + i) * 64] = o[dt][gg][i];
+      }
+    }
+    __syncthreads();
+    if (!late) {
+#pragma unroll
+      for (int gg = 0; gg < NG; ++gg) {
+        const float mo = mine[(34 * gg) * 64], lo = mine[(34 * gg + 1) * 64];
+        const float m = fmaxf(m_run[gg], mo);  // -inf only where no key of either half was visible
+        const float fs = m_run[gg] == -INFINITY ? 0.f : exp2f(m_run[gg] - m);
+        const float fo = mo == -INFINITY ? 0.f : exp2f(mo - m);
+        m_run[gg] = m;
+        l_run[gg] = l_run[gg] * fs + lo * fo;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            o[dt][gg][i] = o[dt][gg][i] * fs + mine[(34 * gg + 2 + 4 * dt + i) * 64] * fo;
+      }
+    }
+  }
+  const bool writes = active && !(PAIR && late);
 
   // ---------------------------------------------------------------- output / split-K hand-off
   // out rows aligned for 4-element stores (16 bytes fp32, 8 bytes fp16 / bf16)
   const bool ovec = (uintptr_t)a.out % 16 == 0 && a.out_row_stride % 4 == 0;
   if (nparts == 1) {
-    if (qvalid) {
+    if (writes) {
 #pragma unroll
-      for (int gg = 0; gg < G; ++gg) {
+      for (int gg = 0; gg < NG; ++gg) {
+        const int qj = qa + 16 * qg(gg) + n;
+        if (qj >= qe) continue;
         const float inv = 1.f / l_run[gg];
-        const int64_t ob = (int64_t)(q0 + qj) * a.out_row_stride + (int64_t)(h * G + gg) * kD;
+        const int64_t ob = (int64_t)(q0 + qj) * a.out_row_stride + (int64_t)(h * G + hd(gg)) * kD;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt)
           store_act4(a.out, a.out_dtype, ob + 16 * dt + 4 * gq, o[dt][gg] * inv, ovec);
@@ -683,15 +740,16 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     }
     return;
   }
-  // Partials of split sp: O rows [G * kAQ][kD] (16-byte stores), then (m, l) per row.
-  constexpr int kRows = G * kAQ;
+  // Partials of split sp: O rows [G * AQ][kD] (16-byte stores), then (m, l) per row.
+  constexpr int kRows = G * AQ;
   const int64_t pstride = (int64_t)kRows * (kD + 2);
   float* po = a.ws_part + ((int64_t)item * a.nsplit + sp) * pstride;
   float* pml = po + (int64_t)kRows * kD;
-  if (qvalid) {
+  if (writes) {
 #pragma unroll
-    for (int gg = 0; gg < G; ++gg) {
-      const int row = gg * kAQ + 16 * wv + n;
+    for (int gg = 0; gg < NG; ++gg) {
+      const int row = hd(gg) * AQ + 16 * qg(gg) + n;
+      if (qa + 16 * qg(gg) + n >= qe) continue;
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) store_agent16(&po[(int64_t)row * kD + 16 * dt + 4 * gq], o[dt][gg]);
       if (gq == 0) store_agent8(&pml[2 * row], float2v{m_run[gg], l_run[gg]});
@@ -716,7 +774,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
   const int nq = qe - qa;
   float* wsm = (float*)&S.t[0];  // [nparts][kRows], nparts <= kMaxParts (host-bounded)
   for (int row = tid; row < kRows; row += kAThreads) {
-    if (row % kAQ >= nq) continue;
+    if (row % AQ >= nq) continue;
     float M = -INFINITY;
     for (int c = 0; c < nparts; ++c) M = fmaxf(M, pbase[c * pstride + (int64_t)kRows * kD + 2 * row]);
     float L = 0.f;
@@ -739,7 +797,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
       acc[u] = float4v{0.f, 0.f, 0.f, 0.f};
       const int it = min(i0 + u * kAThreads, nout - 1);
       const int rr = it >> 5;  // gg * nq + qq
-      rowv[u] = (rr / nq) * kAQ + rr % nq;
+      rowv[u] = (rr / nq) * AQ + rr % nq;
     }
     for (int c = 0; c < nparts; ++c) {
       float4v x[4];
@@ -755,7 +813,7 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     for (int u = 0; u < 4; ++u) {
       const int it = i0 + u * kAThreads;
       if (it >= nout) continue;
-      const int gg = rowv[u] / kAQ, qq = rowv[u] % kAQ;
+      const int gg = rowv[u] / AQ, qq = rowv[u] % AQ;
       const int64_t ob = (int64_t)(q0 + qa + qq) * a.out_row_stride + (int64_t)(h * G + gg) * kD +
                          4 * (it & 31);
       store_act4(a.out, a.out_dtype, ob, acc[u], ovec);
@@ -956,20 +1014,20 @@ namespace ttkv {
 
 namespace {
 
-// Where the two-launch path applies: chunks of more than one 64-query block, G <= 3 (the attend
-// kernel's fragments for 16 queries x G heads fit 256 registers per lane), r1 <= 128.
-bool continuation_eligible(const Geom& g, int G, int max_q_len) {
+// Where the two-launch path applies: chunks of two or more queries, r1 <= 128, and up to max_G
+// query heads per KV head (4 for the attention, 3 for the score tensor: the shapes built).
+bool continuation_eligible(const Geom& g, int G, int max_q_len, int max_G) {
   // every chunk of two or more queries: at 4 x 7,656 keys two launches beat the fused kernel
   // from Q = 2 (137 against 147 us) to Q = 64 (169 against 327 us)
-  return max_q_len > 1 && G >= 1 && G <= 3 && g.r1 <= 128;
+  return max_q_len > 1 && G >= 1 && G <= max_G && g.r1 <= 128;
 }
 
 int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 // Rows per launch: one arrival counter per (row, head, query block), and at most 1 GiB of
 // expanded tiles.
-int cont_slice_reqs(const Geom& g, int num_reqs, int max_q_len, int max_seq_len) {
-  const int n_qb = ceil_div(max_q_len, kAQ);
+int cont_slice_reqs(const Geom& g, int G, int num_reqs, int max_q_len, int max_seq_len) {
+  const int n_qb = ceil_div(max_q_len, attend_queries(G));
   const int64_t per_row = (int64_t)g.H * ceil_div(max_seq_len, kXTile) * kTileBytes;
   const int by_tiles = (int)std::max<int64_t>(1, ((int64_t)1 << 30) / std::max<int64_t>(per_row, 1));
   return std::max(1, std::min({num_reqs, kMaxCounters / (g.H * n_qb), by_tiles}));
@@ -994,11 +1052,11 @@ struct ContShape {
 ContShape cont_shape(const Geom& g, int G, int nr, int max_q_len, int max_seq_len) {
   ContShape s{};
   s.ntl = ceil_div(max_seq_len, kXTile);
-  s.n_qb = ceil_div(max_q_len, kAQ);
+  s.n_qb = ceil_div(max_q_len, attend_queries(G));
   const int items = nr * g.H * s.n_qb;
   s.kchunk = cont_kchunk(items, max_seq_len);
   s.nsplit = std::max(1, ceil_div(max_seq_len, s.kchunk));
-  s.part_bytes = s.nsplit > 1 ? (int64_t)items * s.nsplit * G * kAQ * (kD + 2) * 4 : 0;
+  s.part_bytes = s.nsplit > 1 ? (int64_t)items * s.nsplit * G * attend_queries(G) * (kD + 2) * 4 : 0;
   s.tile_bytes = (int64_t)nr * g.H * s.ntl * kTileBytes;
   return s;
 }
@@ -1038,7 +1096,7 @@ int launch_expand(const ExpandArgs& a, int ksteps, int grid, hipStream_t st) {
 template <int G>
 int launch_attend_t(const AttendArgs& a, int grid, hipStream_t st) {
   const size_t smem = sizeof(AttendSmem);
-  auto kfn = attend_kernel<G>;
+  auto kfn = a.max_q <= attend_queries(G) / 2 ? attend_kernel<G, true> : attend_kernel<G, false>;
   if (int rc = raise_smem_limit((const void*)kfn, smem)) return rc;
   hipLaunchKernelGGL(kfn, dim3(grid), dim3(kAThreads), smem, st, a);
   const hipError_t e = hipGetLastError();
@@ -1103,7 +1161,7 @@ int expand_rows(const Geom& g, const uint8_t* page, int64_t n_slots, int64_t slo
 
 int64_t continuation_scores_workspace_bytes(const Geom& g, int G, int max_q_len,
                                             int max_seq_len) {
-  if (!continuation_eligible(g, G, max_q_len)) return 0;
+  if (!continuation_eligible(g, G, max_q_len, 3)) return 0;
   return (int64_t)g.H * ceil_div(max_seq_len, kXTile) * kTileBytes;
 }
 
@@ -1164,13 +1222,13 @@ int continuation_scores(const Geom& g, int HQ, float scale, const void* q, int q
 }
 
 bool continuation_applies(const Geom& g, int G, int max_q_len) {
-  return continuation_eligible(g, G, max_q_len);
+  return continuation_eligible(g, G, max_q_len, 4);
 }
 
 int64_t continuation_workspace_bytes(const Geom& g, int G, int num_reqs, int max_q_len,
                                      int max_seq_len) {
   if (num_reqs <= 0 || max_q_len <= 0) return 0;
-  const int slice = cont_slice_reqs(g, num_reqs, max_q_len, max_seq_len);
+  const int slice = cont_slice_reqs(g, G, num_reqs, max_q_len, max_seq_len);
   int64_t need = 0;
   for (int nr : {slice, (num_reqs - 1) % slice + 1}) {
     const ContShape s = cont_shape(g, G, nr, max_q_len, max_seq_len);
@@ -1191,7 +1249,7 @@ int continuation_paged(const Geom& g, int HQ, float scale, const void* q, int q_
                        void* out, int out_dtype, int64_t out_row_stride, void* ws, int32_t* err,
                        hipStream_t st) {
   const int G = HQ / g.H;
-  const int slice = cont_slice_reqs(g, num_reqs, max_q_len, max_seq_len);
+  const int slice = cont_slice_reqs(g, G, num_reqs, max_q_len, max_seq_len);
   for (int ri0 = 0; ri0 < num_reqs; ri0 += slice) {
     const int nr = std::min(slice, num_reqs - ri0);
     const ContShape s = cont_shape(g, G, nr, max_q_len, max_seq_len);
@@ -1240,7 +1298,8 @@ int continuation_paged(const Geom& g, int HQ, float scale, const void* q, int q_
       case 1: rc = launch_attend_t<1>(b, grid, st); break;
       case 2: rc = launch_attend_t<2>(b, grid, st); break;
       case 3: rc = launch_attend_t<3>(b, grid, st); break;
-      default: rc = host_fail(TTKV_E_UNSUPPORTED, "attend: G > 3");
+      case 4: rc = launch_attend_t<4>(b, grid, st); break;
+      default: rc = host_fail(TTKV_E_UNSUPPORTED, "attend: G > 4");
     }
     if (rc != TTKV_OK) return rc;
   }
