@@ -32,8 +32,16 @@ class Layout(ctypes.Structure):
 
     @classmethod
     def of(cls, lay) -> "Layout":
-        return cls(lay.H, lay.d, lay.r1, lay.qbits, lay.res_k, lay.res_bits, lay.v_lanes,
-                   lay.v_bits)
+        """The C struct of a layout, kept with it (its fields are frozen, and the library only
+        reads the struct)."""
+        c = lay.__dict__.get("_c_struct")
+        if c is None:
+            c = cls(lay.H, lay.d, lay.r1, lay.qbits, lay.res_k, lay.res_bits, lay.v_lanes,
+                    lay.v_bits)
+            if getattr(type(lay), "__dataclass_params__", None) is not None \
+                    and type(lay).__dataclass_params__.frozen:
+                lay.__dict__["_c_struct"] = c
+        return c
 
 
 def lib_path() -> pathlib.Path:
@@ -181,7 +189,13 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what} failed (code {rc}): {msg}")
 
 
+# the current stream's handle without building a Stream object (a third of a wrapper's host time)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

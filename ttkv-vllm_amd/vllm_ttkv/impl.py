@@ -35,6 +35,7 @@ from __future__ import annotations
 
 import logging
 import os
+import sys
 from dataclasses import dataclass
 
 import torch
@@ -60,18 +61,26 @@ MAX_LEN_ENV = "VLLM_TTKV_MAX_MODEL_LEN"
 DEFAULT_MAX_SEQS = 256
 
 
+_NO_VLLM = False
+
+
 def serving_limits(fallback_len: int | None = None) -> tuple[int, int | None]:
     """(max_num_seqs, max_model_len) the fixed buffers are sized for: the environment
     (`VLLM_TTKV_MAX_NUM_SEQS`, `VLLM_TTKV_MAX_MODEL_LEN`) over the running vLLM config, else 256
     sequences and `fallback_len` (the RoPE table's length: no position beyond it has an angle)."""
+    global _NO_VLLM
     seqs = lens = None
-    try:  # pragma: no cover - vLLM is not installed in the build container
-        from vllm.config import get_current_vllm_config
-        vc = get_current_vllm_config()
-        seqs = getattr(getattr(vc, "scheduler_config", None), "max_num_seqs", None)
-        lens = getattr(getattr(vc, "model_config", None), "max_model_len", None)
-    except Exception:  # noqa: BLE001
-        pass
+    if not _NO_VLLM:
+        try:
+            from vllm.config import get_current_vllm_config
+            vc = get_current_vllm_config()
+            seqs = getattr(getattr(vc, "scheduler_config", None), "max_num_seqs", None)
+            lens = getattr(getattr(vc, "model_config", None), "max_model_len", None)
+        except ModuleNotFoundError as e:
+            # every layer of every step asks: a package that is not installed is looked for once
+            _NO_VLLM = (e.name or "").split(".")[0] == "vllm" and "vllm" not in sys.modules
+        except Exception:  # noqa: BLE001
+            pass
     seqs = int(os.environ.get(MAX_SEQS_ENV) or seqs or DEFAULT_MAX_SEQS)
     lens = os.environ.get(MAX_LEN_ENV) or lens or fallback_len
     return seqs, (None if lens is None else int(lens))
@@ -114,7 +123,7 @@ _WORKSPACES: dict = {}
 
 def _capturing() -> bool:
     """Is the current stream recording a graph? (False where there is no device.)"""
-    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
 
 def workspaces(device) -> DeviceWorkspaces:
@@ -363,6 +372,9 @@ class TTKVAttentionImpl(_ImplBase):
         g = _hip.Layout.of(lay)
         need = L.ttkv_decode_workspace_bytes(g, self.num_heads, num_reqs, max_seq_len, block_size)
         seqs, lens = self._limits
+        buf = workspaces(device).bufs.get("decode")
+        if buf is not None and buf.numel() >= need:
+            return buf
         cap = L.ttkv_decode_workspace_bytes(g, self.num_heads, max(seqs, num_reqs),
                                             max(lens or 0, max_seq_len), block_size)
         return workspaces(device).get("decode", need, cap, fixed=True)
@@ -372,6 +384,9 @@ class TTKVAttentionImpl(_ImplBase):
         g = _hip.Layout.of(lay)
         need = L.ttkv_write_workspace_bytes(g, num_tokens)
         if fixed:   # a decode step's tokens: one per sequence
+            buf = workspaces(device).bufs.get("decode_write")
+            if buf is not None and buf.numel() >= need:
+                return buf
             cap = L.ttkv_write_workspace_bytes(g, max(self._limits[0], num_tokens))
             return workspaces(device).get("decode_write", need, cap, fixed=True)
         return workspaces(device).get("prefill_write", need)

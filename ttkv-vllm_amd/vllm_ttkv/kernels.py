@@ -14,9 +14,10 @@ from .layout import TTKLayout
 
 
 def _need_device(*ts):
-    ts = [u for t in ts for u in (t if isinstance(t, DecoderPool) else (t,))]
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if isinstance(t, DecoderPool):
+            _need_device(*t)
+        elif t is not None and not t.is_cuda:
             raise RuntimeError("libttkv_hip kernels take device tensors; got a "
                                f"{t.device.type} tensor (there is no CPU implementation)")
 
@@ -36,12 +37,12 @@ def pool_args(lay: TTKLayout, dec_pool: DecoderPool) -> tuple[int, int, int]:
                         "decoder_pool.pack_decoders of fp32 decoders)")
     q, sc = dec_pool
     R = decoder_ranks(lay.r1)
-    if (q.dtype != torch.int8 or q.dim() != 3 or tuple(q.shape[1:]) != (lay.H * lay.d, R)
+    if (q.dtype != torch.int8 or q.dim() != 3 or q.shape[1:] != (lay.H * lay.d, R)
             or not q.is_contiguous()):
         raise ValueError(f"dec_pool.q must be contiguous int8 [slots, {lay.H * lay.d}, {R}], got "
                          f"{q.dtype} {tuple(q.shape)} (a decoder written at one rank cannot be "
                          f"read at another)")
-    if sc.dtype != torch.float32 or tuple(sc.shape) != (q.shape[0], R) or not sc.is_contiguous():
+    if sc.dtype != torch.float32 or sc.shape != (q.shape[0], R) or not sc.is_contiguous():
         raise ValueError(f"dec_pool.scale must be contiguous fp32 [{q.shape[0]}, {R}], got "
                          f"{sc.dtype} {tuple(sc.shape)}")
     return q.data_ptr(), sc.data_ptr(), int(q.shape[0])
@@ -58,6 +59,18 @@ def page_bytes(page: torch.Tensor, blob: int) -> torch.Tensor:
     if not u8.is_contiguous():
         raise ValueError("the cache page must be contiguous")
     return u8.reshape(-1, u8.shape[-1])
+
+
+def _page_args(page: torch.Tensor, blob: int) -> tuple[int, int, int]:
+    """(pointer, slots, bytes per slot) of a paged cache, as `page_bytes` views it (the same
+    refusals, without making the views)."""
+    if page.dim() < 2 or not page.is_contiguous():
+        flat = page_bytes(page, blob)
+        return flat.data_ptr(), flat.shape[0], flat.stride(0)
+    row = page.shape[-1] * page.element_size()
+    if row < blob:
+        raise ValueError(f"the cache row is {row} bytes but the layout needs {blob}")
+    return page.data_ptr(), page.numel() // max(page.shape[-1], 1), row
 
 
 def decode_workspace(lay: TTKLayout, num_heads: int, num_reqs: int, max_seq_len: int,
@@ -94,8 +107,7 @@ def decode_paged(lay: TTKLayout, query: torch.Tensor, page: torch.Tensor, block_
         raise ValueError(f"query head dim {d} != layout d {lay.d}")
     if query.stride(2) != 1 or query.stride(1) != d:
         raise ValueError("query must be contiguous within a token ([HQ, d] rows)")
-    blob = lay.compressed_bytes_per_token()
-    flat = page_bytes(page, blob)
+    page_ptr, n_slots, slot_bytes = _page_args(page, lay.compressed_bytes_per_token())
     _i32(block_table, "block_table")
     _i32(seq_lens, "seq_lens")
     _i32(query_start_loc, "query_start_loc")
@@ -120,7 +132,7 @@ def decode_paged(lay: TTKLayout, query: torch.Tensor, page: torch.Tensor, block_
     rc = L.ttkv_decode_paged(
         _hip.Layout.of(lay), HQ, float(scale),
         query.data_ptr(), _hip.DTYPE_CODE[query.dtype], query.stride(0),
-        flat.data_ptr(), flat.shape[0], flat.stride(0),
+        page_ptr, n_slots, slot_bytes,
         int(block_size), block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
         seq_lens.data_ptr(), query_start_loc.data_ptr(), num_reqs, int(max_seq_len),
         dec_slot_of_block.data_ptr(), dec_slot_of_block.numel(), dq, ds, n_dec,
@@ -166,9 +178,9 @@ def write_paged(lay: TTKLayout, key: torch.Tensor, value: torch.Tensor,
     _i32(dec_slot_of_block, "dec_slot_of_block")
     dq, ds, n_dec = pool_args(lay, dec_pool)
     if pinv_pool is not None and (pinv_pool.dtype != torch.float32 or
-                                  tuple(pinv_pool.shape[1:]) != (lay.r1, lay.H * lay.d)):
+                                  pinv_pool.shape[1:] != (lay.r1, lay.H * lay.d)):
         raise ValueError("pinv_pool must be fp32 [slots, r1, H*d] (each pinv transposed)")
-    flat = page_bytes(page, lay.compressed_bytes_per_token())
+    page_ptr, n_slots, slot_bytes = _page_args(page, lay.compressed_bytes_per_token())
     if error_word is None:
         error_word = torch.zeros(1, dtype=torch.int32, device=key.device)
     if dec_used is not None:
@@ -192,8 +204,7 @@ def write_paged(lay: TTKLayout, key: torch.Tensor, value: torch.Tensor,
         slot_mapping.data_ptr(), N, query_start_loc.data_ptr(), query_start_loc.numel() - 1,
         block_table.data_ptr(), block_table.stride(0), dec_slot_of_block.data_ptr(),
         dec_slot_of_block.numel(), dq, ds, _hip.ptr(pinv_pool), n_dec,
-        _hip.ptr(dec_used), _hip.ptr(cq), _hip.ptr(coeff_scale_in), flat.data_ptr(),
-        flat.shape[0], flat.stride(0),
+        _hip.ptr(dec_used), _hip.ptr(cq), _hip.ptr(coeff_scale_in), page_ptr, n_slots, slot_bytes,
         _hip.ptr(coeff_out), _hip.ptr(resid_out), _hip.ptr(workspace),
         0 if workspace is None else workspace.numel(), error_word.data_ptr(),
         _hip.stream_ptr(key.device))

@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
+from functools import cached_property
 
 import torch
 
@@ -135,6 +136,11 @@ class TTKLayout:
         return 2 * self.H * self.d * 2
 
     def compressed_bytes_per_token(self) -> int:
+        return self._blob_bytes
+
+    @cached_property
+    def _blob_bytes(self) -> int:
+        # (the fields are frozen; the kernels' wrappers ask for this on every call)
         return self.k_slot_bytes + self.v_slot_bytes
 
     def ratio(self) -> float:
