@@ -773,19 +773,56 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
   const float* pbase = a.ws_part + (int64_t)item * a.nsplit * pstride;
   const int nq = qe - qa;
   float* wsm = (float*)&S.t[0];  // [nparts][kRows], nparts <= kMaxParts (host-bounded)
-  for (int row = tid; row < kRows; row += kAThreads) {
-    if (row % AQ >= nq) continue;
-    float M = -INFINITY;
-    for (int c = 0; c < nparts; ++c) M = fmaxf(M, pbase[c * pstride + (int64_t)kRows * kD + 2 * row]);
-    float L = 0.f;
-    for (int c = 0; c < nparts; ++c) {
-      const float* ml = pbase + c * pstride + (int64_t)kRows * kD + 2 * row;
-      const float e = ml[0] == -INFINITY ? 0.f : exp2f(ml[0] - M);
-      L = fmaf(ml[1], e, L);
-      wsm[c * kRows + row] = e;
+  if constexpr (PAIR) {
+    // Short chunks have many splits of few rows: the (m, l) of 16 splits per round trip (2 queries
+    // over 7,656 keys: 60 -> 54 us). The long chunks' kernel has no registers left for it, and
+    // few splits.
+    for (int row = tid; row < kRows; row += kAThreads) {
+      if (row % AQ >= nq) continue;
+      const float* ml0 = pbase + (int64_t)kRows * kD + 2 * row;
+      float M = -INFINITY;
+      for (int c0 = 0; c0 < nparts; c0 += 16) {
+        float m[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m[i] = *gbl(ml0 + min(c0 + i, nparts - 1) * pstride);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          M = fmaxf(M, m[i]);
+          if (c0 + i < nparts) wsm[(c0 + i) * kRows + row] = m[i];
+        }
+      }
+      float L = 0.f;
+      for (int c0 = 0; c0 < nparts; c0 += 16) {
+        float l[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) l[i] = *gbl(ml0 + min(c0 + i, nparts - 1) * pstride + 1);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          if (c0 + i >= nparts) continue;
+          const float m = wsm[(c0 + i) * kRows + row];
+          const float e = m == -INFINITY ? 0.f : exp2f(m - M);
+          L = fmaf(l[i], e, L);
+          wsm[(c0 + i) * kRows + row] = e;
+        }
+      }
+      const float inv = 1.f / L;
+      for (int c = 0; c < nparts; ++c) wsm[c * kRows + row] *= inv;
     }
-    const float inv = 1.f / L;
-    for (int c = 0; c < nparts; ++c) wsm[c * kRows + row] *= inv;
+  } else {
+    for (int row = tid; row < kRows; row += kAThreads) {
+      if (row % AQ >= nq) continue;
+      float M = -INFINITY;
+      for (int c = 0; c < nparts; ++c) M = fmaxf(M, pbase[c * pstride + (int64_t)kRows * kD + 2 * row]);
+      float L = 0.f;
+      for (int c = 0; c < nparts; ++c) {
+        const float* ml = pbase + c * pstride + (int64_t)kRows * kD + 2 * row;
+        const float e = ml[0] == -INFINITY ? 0.f : exp2f(ml[0] - M);
+        L = fmaf(ml[1], e, L);
+        wsm[c * kRows + row] = e;
+      }
+      const float inv = 1.f / L;
+      for (int c = 0; c < nparts; ++c) wsm[c * kRows + row] *= inv;
+    }
   }
   __syncthreads();
   const int nout = G * nq * (kD / 4);
