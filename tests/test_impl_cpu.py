@@ -350,3 +350,16 @@ def test_serving_limits_from_environment(monkeypatch):
     monkeypatch.setenv("VLLM_TTKV_MAX_NUM_SEQS", "12")
     monkeypatch.setenv("VLLM_TTKV_MAX_MODEL_LEN", "777")
     assert impl.serving_limits(1234) == (12, 777)
+
+
+def test_serving_limits_from_a_config_loaded_later(monkeypatch):
+    """A call that found no vllm does not hide one that is loaded after it."""
+    from types import SimpleNamespace
+    monkeypatch.delenv("VLLM_TTKV_MAX_NUM_SEQS", raising=False)
+    monkeypatch.delenv("VLLM_TTKV_MAX_MODEL_LEN", raising=False)
+    assert impl.serving_limits(1234) == (256, 1234)
+    vc = SimpleNamespace(scheduler_config=SimpleNamespace(max_num_seqs=31),
+                         model_config=SimpleNamespace(max_model_len=99))
+    monkeypatch.setitem(__import__("sys").modules, "vllm.config",
+                        SimpleNamespace(get_current_vllm_config=lambda: vc))
+    assert impl.serving_limits(1234) == (31, 99)

@@ -70,14 +70,15 @@ def serving_limits(fallback_len: int | None = None) -> tuple[int, int | None]:
     sequences and `fallback_len` (the RoPE table's length: no position beyond it has an angle)."""
     global _NO_VLLM
     seqs = lens = None
-    if not _NO_VLLM:
+    if not _NO_VLLM or "vllm" in sys.modules or "vllm.config" in sys.modules:
         try:
             from vllm.config import get_current_vllm_config
             vc = get_current_vllm_config()
             seqs = getattr(getattr(vc, "scheduler_config", None), "max_num_seqs", None)
             lens = getattr(getattr(vc, "model_config", None), "max_model_len", None)
         except ModuleNotFoundError as e:
-            # every layer of every step asks: a package that is not installed is looked for once
+            # every layer of every step asks: a package that is not installed is searched for
+            # once, and found again as soon as a module of that name is loaded
             _NO_VLLM = (e.name or "").split(".")[0] == "vllm" and "vllm" not in sys.modules
         except Exception:  # noqa: BLE001
             pass
