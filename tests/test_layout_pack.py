@@ -3,7 +3,9 @@ slot bytes the REFERENCE wrote (tests/golden/ref_encode_*.npz: `fit_k_slots`, `f
 `v_slots`, with the coefficients and rulers they were packed from), against the oracle's packer
 on random row stores, and by round trips. Reference: vllm_ttkv/layout.py:161-261 and its test
 tests/test_layout.py (pack, then unpack, must be a faithful rearrangement)."""
+import copy
 import pathlib
+import pickle
 from types import SimpleNamespace
 
 import numpy as np
@@ -11,7 +13,7 @@ import pytest
 import torch
 
 from oracle import layout as olayout
-from vllm_ttkv import layout as play
+from vllm_ttkv import _hip, layout as play
 
 GOLD = pathlib.Path(__file__).resolve().parent / "golden"
 
@@ -87,3 +89,15 @@ def test_pack_refuses_a_row_count_that_is_not_h_times_n():
         play.pack_k_slots(lay, torch.zeros(3, 110, dtype=torch.int8), torch.zeros(3), rows)
     with pytest.raises(ValueError):
         play.pack_v_slots(lay, rows)
+
+
+def test_copies_hold_the_fields_alone():
+    """What the kernels' wrappers keep with a layout stays out of its copies and pickles."""
+    lay = play.layout_for_config(play.CONFIGS["safe"], 110)
+    fresh = pickle.dumps(lay)
+    lay.compressed_bytes_per_token()
+    _hip.Layout.of(lay)
+    assert pickle.dumps(lay) == fresh
+    for twin in (pickle.loads(fresh), copy.copy(lay), copy.deepcopy(lay)):
+        assert twin == lay and "_c_struct" not in twin.__dict__
+        assert twin.compressed_bytes_per_token() == lay.compressed_bytes_per_token()

@@ -23,7 +23,7 @@ store as separate row arrays.
 from __future__ import annotations
 
 import math
-from dataclasses import dataclass
+from dataclasses import dataclass, fields
 from functools import cached_property
 
 import torch
@@ -137,6 +137,10 @@ class TTKLayout:
 
     def compressed_bytes_per_token(self) -> int:
         return self._blob_bytes
+
+    def __getstate__(self) -> dict:
+        # copies and pickles hold the fields alone, not what is kept beside them
+        return {f.name: getattr(self, f.name) for f in fields(self)}
 
     @cached_property
     def _blob_bytes(self) -> int:
