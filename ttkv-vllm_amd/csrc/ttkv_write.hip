@@ -642,7 +642,7 @@ __global__ __launch_bounds__(kPThreads, 6) void pack_tiles_kernel(WriteArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __syncthreads();
-  // ---- the decoder's part of the keys: rec[token][dim], dims 32w .. 32w + 31 in this wave
+  // ---- the decoder's part of the keys: rec[token][dim], dims 16w .. 16w + 15 in this wave
   float4v rec = {0.f, 0.f, 0.f, 0.f};  // dims 16w + 4gq .. + 3 of token n
   const int ds_n = __shfl(ds, n);
   for (uint64_t todo = ok; todo;) {  // one pass per distinct decoder, alike in every wave
