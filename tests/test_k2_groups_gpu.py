@@ -54,3 +54,29 @@ def test_row_groups(cfg, H, G, r1, dtype, lens, qlens):
     for r in range(len(lens)):
         e = (first[qsl[r]:qsl[r + 1]].double() - want[r]).abs()
         assert e.max() <= tol * 2e-3 and e.mean() <= tol * 1e-3, (r, e.max(), e.mean())
+
+
+def test_four_heads_with_a_workspace_too_small_for_tiles():
+    """Four query heads per KV head and a workspace that holds no expanded tiles: the fused kernel,
+    whose keys are not split here."""
+    st = fitted_store("safe", 200, seed=51)
+    pg = paged([st], 16, 4)
+    q = synth.queries(40, HQ=32, seed=10, dtype=torch.float16)
+    qsl = torch.tensor([0, 40], dtype=torch.int32)
+    cache = llama3_cache(512)
+    dev = "cuda"
+    dec_map = torch.full((pg["num_blocks"],), -1, dtype=torch.int32)
+    dec_map[pg["block_table"][0, 0]] = 0
+    out = torch.full((40, 32, 128), float("nan"), dtype=torch.float16, device=dev)
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    kernels.prefill_paged(st["lay"], q.to(dev), pg["page"].to(dev), 16,
+                          pg["block_table"].to(dev), pg["seq_lens"].to(dev), qsl.to(dev), 40, 200,
+                          dec_map.to(dev), dec_pool_of([st["decoder"]], dev), cache.to(dev), SCALE,
+                          out=out, error_word=err,
+                          workspace=torch.zeros(256, dtype=torch.uint8, device=dev))
+    torch.cuda.synchronize()
+    want = attend.paged_continuation(st["lay"], pg["page"], pg["block_table"], pg["seq_lens"], qsl,
+                                     q.float(), [st["decoder"]], cache, 16, SCALE,
+                                     dtype=torch.float64)[0]
+    e = (out.float().cpu().double() - want).abs()
+    assert int(err.item()) == 0 and e.max() <= 2e-3 and e.mean() <= 1e-3

@@ -725,16 +725,21 @@ static int64_t prefill_part_bytes(const Geom& g, int G, int nr, int max_q_len, i
   return (int64_t)items * nsplit * G * kPQ * (kD + 2) * 4;
 }
 
-int64_t prefill_workspace_bytes(const Geom& g, int G, int num_reqs, int max_q_len,
-                                int max_seq_len, int block_size) {
+static int64_t fused_workspace_bytes(const Geom& g, int G, int num_reqs, int max_q_len,
+                                     int max_seq_len, int block_size) {
   if (num_reqs <= 0 || max_q_len <= 0) return 0;
-  if (continuation_applies(g, G, max_q_len))
-    return continuation_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len);
   const int slice = prefill_slice_reqs(g, num_reqs, max_q_len);
   const int64_t part = std::max(
       prefill_part_bytes(g, G, slice, max_q_len, max_seq_len, block_size),
       prefill_part_bytes(g, G, (num_reqs - 1) % slice + 1, max_q_len, max_seq_len, block_size));
   return part ? kCounterBytes + part : 0;
+}
+
+int64_t prefill_workspace_bytes(const Geom& g, int G, int num_reqs, int max_q_len,
+                                int max_seq_len, int block_size) {
+  if (num_reqs > 0 && continuation_applies(g, G, max_q_len))
+    return continuation_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len);
+  return fused_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len, block_size);
 }
 
 int prefill_paged(const Geom& g, int HQ, float scale, const void* q, int q_dtype,
@@ -830,16 +835,25 @@ int prefill_paged(const Geom& g, int HQ, float scale, const void* q, int q_dtype
   if ((int64_t)g.H * a.n_qb > kMaxCounters)
     return host_fail(TTKV_E_UNSUPPORTED, "max_q_len=" + std::to_string(max_q_len) +
                                              " is past the longest query chunk built");
+  bool expand = !scores && continuation_applies(g, G, max_q_len);
   if (!scores) {
-    const int64_t need = prefill_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len, block_size);
+    int64_t need = prefill_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len, block_size);
+    // Four query heads per KV head: a workspace that cannot hold the expanded tiles serves the fused
+    // kernel (of the other shapes with two launches such a call is refused).
+    if (expand && G == 4 && (!ws || ws_bytes < need || (uintptr_t)ws % 256)) {
+      const int64_t fused =
+          fused_workspace_bytes(g, G, num_reqs, max_q_len, max_seq_len, block_size);
+      if (ws ? ws_bytes >= fused : fused == 0) {
+        expand = false;
+        need = fused;
+      }
+    }
     if (need && (!ws || ws_bytes < need))
       return host_fail(TTKV_E_WORKSPACE, "prefill workspace needs " + std::to_string(need) +
                                              " bytes, got " + std::to_string(ws_bytes));
     if (need && (uintptr_t)ws % 256)
       return host_fail(TTKV_E_INVALID, "workspace not 256-byte aligned");
   }
-  // chunks of more than one 64-query block: every key expanded once, then attended by all the
-  // chunk's queries (ttkv_continuation.hip)
   // the score tensor of a long chunk from the expanded tiles, when the caller gave a workspace
   // for them (without one, the fused kernel below)
   if (scores && ws) {
@@ -851,7 +865,9 @@ int prefill_paged(const Geom& g, int HQ, float scale, const void* q, int q_dtype
                                  n_dec_slots, cs_cache, s_out, s_head_stride, s_q_stride, ws, err,
                                  st);
   }
-  if (!scores && continuation_applies(g, G, max_q_len))
+  // chunks of two or more queries: every key expanded once, then attended by all the chunk's queries
+  // (ttkv_continuation.hip)
+  if (expand)
     return continuation_paged(g, HQ, scale, q, q_dtype, q_row_stride, page, n_slots, slot_stride,
                               block_size, bt, bt_row_stride, seq_lens, qsl, req_index, num_reqs,
                               max_q_len, max_seq_len, dec_map, num_blocks, dec_q, dec_scale,
