@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from helpers import dec_pool_of, fitted_store, llama3_cache, paged
-from oracle import attend
+from oracle import attend, rope
 from vllm_ttkv import kernels, synth
 
 pytestmark = pytest.mark.gpu
@@ -54,6 +54,38 @@ def test_row_groups(cfg, H, G, r1, dtype, lens, qlens):
     for r in range(len(lens)):
         e = (first[qsl[r]:qsl[r + 1]].double() - want[r]).abs()
         assert e.max() <= tol * 2e-3 and e.mean() <= tol * 1e-3, (r, e.max(), e.mean())
+
+
+@pytest.mark.parametrize("G,n,Q", [(4, 300, 40), (4, 300, 130), (3, 300, 40), (3, 300, 130),
+                                   (1, 200, 70)])
+@pytest.mark.parametrize("scale", [-0.09, 0.0])
+def test_scales_that_are_not_positive(G, n, Q, scale):
+    """A negative scale turns the order of the scores and a zero one makes them alike; the keys
+    past a query stay hidden under both."""
+    print(f"[k2 scale] G={G} n={n} Q={Q} scale={scale}", flush=True)
+    st = fitted_store("safe", n, seed=60)
+    pg = paged([st], 16, 4)
+    q = synth.queries(Q, HQ=8 * G, seed=11, dtype=torch.float16)
+    qsl = torch.tensor([0, Q], dtype=torch.int32)
+    cache = llama3_cache(512)
+    dev = "cuda"
+    dec_map = torch.full((pg["num_blocks"],), -1, dtype=torch.int32)
+    dec_map[pg["block_table"][0, 0]] = 0
+    out = kernels.prefill_paged(st["lay"], q.to(dev), pg["page"].to(dev), 16,
+                                pg["block_table"].to(dev), pg["seq_lens"].to(dev), qsl.to(dev), Q, n,
+                                dec_map.to(dev), dec_pool_of([st["decoder"]], dev), cache.to(dev),
+                                scale)
+    lay = st["lay"]
+    ks, vs = attend.gather_request(lay, pg["page"], pg["block_table"][0], n, 16)
+    cos, sin = rope.cos_sin_from_cache(cache, torch.arange(n), 128)
+    s = attend.raw_scores_multi(lay, ks, st["decoder"], q.permute(1, 0, 2), cos, sin, scale,
+                                p0=n - Q, dtype=torch.float64)
+    p = torch.softmax(s, -1)
+    V = attend.dense_v_from_slots(lay, vs, torch.float64).repeat_interleave(G, 0)
+    e = (out.cpu().double().permute(1, 0, 2) - p @ V).abs()
+    # each weight times its row's ruler is rounded to fp16 once, and so is the output: 2^-11 of
+    # sum p |v| each; 1e-4 for the 32-bit scores (|s| < 15)
+    assert (e <= 2.0 ** -10 * (p @ V.abs()) + 1e-4).all(), e.max()
 
 
 def test_four_heads_with_a_workspace_too_small_for_tiles():

@@ -358,7 +358,8 @@ __global__ __launch_bounds__(kXThreads, 2) void expand_kernel(ExpandArgs a) {
 struct AttendArgs {
   Geom g;
   int HQ, G;
-  float scale_log2;
+  float scale_log2;  // > 0: masked raw scores are -inf before they are scaled
+  float q_factor;    // 1, or -1 / 0 for a negative / zero scale: factor of the query
   const void* q;
   int q_dtype;
   int64_t q_row_stride;
@@ -518,7 +519,8 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
         load_act_n<4>(a.q, a.q_dtype, qrow + 16 * ks, qvec, tq);
         load_act_n<4>(a.q, a.q_dtype, qrow + 64 + 16 * ks, qvec, tq + 4);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) qf[gg][ks][i] = qvalid ? (_Float16)tq[i] : (_Float16)0.0f;
+        for (int i = 0; i < 8; ++i)
+          qf[gg][ks][i] = qvalid ? (_Float16)(tq[i] * a.q_factor) : (_Float16)0.0f;
       }
     }
   }
@@ -1301,7 +1303,9 @@ int continuation_paged(const Geom& g, int HQ, float scale, const void* q, int q_
     b.g = g;
     b.HQ = HQ;
     b.G = G;
-    b.scale_log2 = scale * 1.4426950408889634f;
+    // s = scale * q.k = |scale| * (sign(scale) * q).k, exactly; a zero scale zeroes the query
+    b.scale_log2 = scale == 0.f ? 1.f : fabsf(scale) * 1.4426950408889634f;
+    b.q_factor = scale > 0.f ? 1.f : scale < 0.f ? -1.f : 0.f;
     b.q = q;
     b.q_dtype = q_dtype;
     b.q_row_stride = q_row_stride;
