@@ -167,9 +167,11 @@ int ttkv_decode_paged_noalloc(const ttkv_layout* lay, int32_t num_heads, float s
  *   whole rows).
  * Work is spread over two launches: the projection, one workgroup per (token, 4 ranks), each
  * rank's sum complete in its workgroup; then, per (token, KV head), the quantisation (every head
- * alike), the residual and the K and V rows. The tokens past the first num_reqs of a call (a
- * step's decode tokens lie among those; of a single request: all) go in tiles of 16 tokens when
- * they are 192 or more. The projection and each token's decoder slot live in
+ * alike), the residual and the K and V rows. Calls of 208 tokens or more (3 more for every request past
+ * the first) take both launches in tiles of up to 16 tokens of one request. The two ways sum the
+ * projection and the residual in different orders of 32-bit additions: a token's bytes do not
+ * depend on the others of its call, but where a sum lies at a rounding border they can depend on
+ * which way its call was written. The projection and each token's decoder slot live in
  * `workspace` (ttkv_write_workspace_bytes). */
 int ttkv_write_paged(const ttkv_layout* lay, const void* key, int32_t k_dtype, int64_t k_row_stride,
                      const void* value, int32_t v_dtype, int64_t v_row_stride,

@@ -1,5 +1,5 @@
-"""K3 over chunks of tokens (16-token tiles) on the GPU: at the edges of tiles and requests, the
-float stages within the rounding of their own sums against 64 bits, and every byte exactly the
+"""K3 over many tokens (tiles of up to 16 tokens of one request, from 208 tokens on and 3 more for
+every further request) on the GPU: at the edges of tiles and requests, the float stages within the rounding of their own sums against 64 bits, and every byte exactly the
 oracle's from the kernel's own projection and residual."""
 import pytest
 import torch
@@ -23,6 +23,10 @@ def _decoder(r1, H, seed):
     return q * (torch.rand(r1, generator=g) * 0.02 + 0.005).half().float()[:, None]
 
 
+def _tiled(counts):
+    return sum(counts) >= 208 + 3 * (len(counts) - 1)
+
+
 def _case(cfg, r1, H, counts, dtype, seed, fit=False):
     lay = layout_for_config(config_named(cfg), r1=r1, H=H)
     g = torch.Generator().manual_seed(seed)
@@ -43,16 +47,18 @@ def _case(cfg, r1, H, counts, dtype, seed, fit=False):
                 H=H)
 
 
-def _run(c, slots=None, dec_map=None, used=None):
+def _run(c, slots=None, dec_map=None, used=None, views=None, n_slots=None):
     lay, N, B, H = c["lay"], len(c["req"]), len(c["decs"]), c["H"]
-    page = torch.zeros(N + 40, lay.compressed_bytes_per_token(), dtype=torch.uint8, device=DEV)
+    page = torch.zeros(n_slots or N + 40, lay.compressed_bytes_per_token(), dtype=torch.uint8,
+                       device=DEV)
     bt = torch.arange(B, dtype=torch.int32, device=DEV).reshape(B, 1)
     if dec_map is None:
         dec_map = torch.arange(B, dtype=torch.int32)
     c_out = torch.zeros(N, lay.r1, device=DEV)
     r_out = torch.zeros(N, H * D, device=DEV)
     err = torch.zeros(1, dtype=torch.int32, device=DEV)
-    kernels.write_paged(lay, c["K"].reshape(N, H, D).to(DEV), c["V"].reshape(N, H, D).to(DEV),
+    v = views or {n: c[n].reshape(N, H, D).to(DEV) for n in "KV"}
+    kernels.write_paged(lay, v["K"], v["V"],
                         (c["slots"] if slots is None else slots).to(DEV), c["qsl"].to(DEV), bt,
                         dec_map.to(DEV), dec_pool_of(c["decs"], DEV),
                         torch.stack([p.t() for p in c["pinvs"]]).contiguous().to(DEV), page,
@@ -86,19 +92,24 @@ def _want(c, coef, R):
 
 CASES = [
     # (config, r1, KV heads, tokens per request, dtype, from a fit)
-    ("safe", 110, 8, [192], torch.float32, False),            # whole tiles
-    ("safe", 110, 8, [191], torch.float16, False),            # one token short of tiles
-    ("safe", 110, 8, [207], torch.bfloat16, False),           # a 15-token last tile
+    ("safe", 110, 8, [208], torch.float32, False),            # whole tiles
+    ("safe", 110, 8, [207], torch.float16, False),            # one token short of tiles
+    ("safe", 110, 8, [223], torch.bfloat16, False),           # a 15-token last tile
+    ("safe", 110, 8, [192], torch.float32, False),            # token by token
     ("campaign4x", 110, 8, [1, 1, 1, 218], torch.float16, False),  # decodes, then a chunk
-    ("tight", 64, 8, [5, 190, 17], torch.float16, False),      # tiles straddling two requests
-    ("safe", 7, 2, [1] * 20 + [137, 75, 3], torch.float16, False),  # and three; a small rank
-    ("safe", 200, 4, [198], torch.float32, False),             # ranks past 128
+    ("campaign4x", 110, 8, [218, 1, 17, 1], torch.float16, False),  # and behind it
+    ("tight", 64, 8, [5, 200, 17], torch.float16, False),      # partly filled tiles
+    ("tight", 64, 8, [5, 190, 17], torch.float16, False),      # two tokens short of tiles
+    ("safe", 7, 2, [1] * 20 + [187, 75, 3], torch.float16, False),  # a small rank
+    ("safe", 16, 1, [1] * 70 + [400, 0, 3, 2], torch.float16, False),  # spans past one wave's lanes
+    ("safe", 200, 4, [213], torch.float32, False),             # ranks past 128
     ("safe", 96, 3, [209], torch.float16, False),              # H * d / 4 not a multiple of 64
-    ("safe", 110, 1, [193], torch.float16, False),
-    ("safe_fp16", 110, 8, [187, 20], torch.float16, False),
-    ("campaign4x_int4g32", 110, 8, [187, 20], torch.bfloat16, False),
+    ("safe", 110, 1, [209], torch.float16, False),
+    ("safe_fp16", 110, 8, [197, 20], torch.float16, False),
+    ("campaign4x_int4g32", 110, 8, [197, 20], torch.bfloat16, False),
     ("campaign4x_int4g32", 66, 8, [212], torch.float16, False),
     ("safe", 110, 8, [150, 61], torch.float16, True),          # fits' own coefficients
+    ("safe", 16, 1, [100, 16600], torch.float16, False),       # two launches of each kernel
 ]
 
 
@@ -148,3 +159,42 @@ def test_skipped_and_refused_tokens_inside_tiles():
     assert torch.equal(page[c["slots"][keep]], clean[c["slots"][keep]])
     assert int(page[c["slots"][~keep]].abs().sum()) == 0
     assert used.tolist() == [1, 0, 1]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_rows_without_alignment(dtype):
+    """Keys and values as views of wider rows at an odd offset: the bytes of packed ones."""
+    c = _case("safe", 110, 8, [140, 83], dtype, seed=5)
+    assert _tiled([140, 83])
+    want, coef, R, err = _run(c)
+    assert err == 0
+    wide = {}
+    for name in ("K", "V"):
+        x = c[name].to(DEV)
+        buf = torch.zeros(x.shape[0], x.shape[1] + 3, dtype=dtype, device=DEV)
+        buf[:, 1:1 + x.shape[1]] = x
+        wide[name] = buf[:, 1:1 + x.shape[1]].unflatten(1, (8, D))
+        assert wide[name].data_ptr() % 16 and wide[name].stride(0) == 8 * D + 3
+    page, coef2, R2, err = _run(c, views=wide)
+    assert err == 0 and torch.equal(page, want)
+    assert torch.equal(coef2, coef) and torch.equal(R2, R)
+
+
+def test_tokens_outside_every_request():
+    """Tokens before the first request and after the last: refused, or skipped where they are
+    padding; the requests' own bytes are those of a call without them."""
+    c = _case("safe", 110, 8, [100, 125], torch.float16, seed=8)
+    want, _, _, err = _run(c)
+    assert err == 0 and _tiled([100, 125])
+    more = dict(c)
+    for name in ("K", "V"):
+        x = c[name]
+        more[name] = torch.cat([x[:5], x, x[-9:]])
+    more["qsl"] = c["qsl"] + 5
+    used = c["slots"]
+    free = torch.tensor([i for i in range(225 + 40) if i not in set(used.tolist())])
+    for outside, bits in ((torch.full((14,), -1), 0), (free[:14], 1)):
+        slots = torch.cat([outside[:5], used, outside[5:]])
+        page, _, _, err = _run(dict(more, slots=slots, req=torch.zeros(239)), n_slots=265)
+        assert err == bits
+        assert torch.equal(page, want)

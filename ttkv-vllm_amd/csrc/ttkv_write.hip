@@ -1,10 +1,10 @@
-// K3: write/encode of new tokens into compressed slots, one launch for all tokens of a layer.
+// K3: write/encode of new tokens into compressed slots, two launches for all tokens of a layer.
 // gfx950 / CDNA4.
 //
-// Single tokens (a decode step's, one per request): two launches of 256-thread workgroups, so a
-// batch of B tokens spreads its B x 450 KB of pinv and B x 113 KB of decoder reads over many CUs.
-// Chunks of tokens take the same two launches in tiles of 16 tokens (project_tiles_kernel,
-// pack_tiles_kernel), which read a request's pinv and decoder once per tile:
+// Few tokens per request (a decode step has one): 256-thread workgroups per token, so a batch of B
+// tokens spreads its B x 450 KB of pinv and B x 132 KB of decoder reads over many CUs. Calls of more
+// tokens take the same two launches in tiles of up to 16 tokens of one request
+// (project_tiles_kernel, pack_tiles_kernel), which read its pinv and decoder once per tile:
 //   K3a project  one workgroup per (token, 4 ranks): c[a] for its ranks over all H*d
 //             dims, complete in the workgroup (wave sums, fixed order), left in the workspace
 //                                                                  -- skipped when a fit gives (cq, cs)
@@ -65,11 +65,17 @@ struct WriteArgs {
   float* r_out;
   int* err;
   int tok0;         // first token of this launch (tokens tok0 .. tok0 + num_tokens - 1)
-  int n_single;     // its first n_single tokens are done one by one, the rest in 16-token tiles
+  int tiles;        // at most so many tiles hold its tokens (tiled launches)
   float* ws_c;      // [num_tokens][r1] each token's projection c, from K3a for K3b
   int* ws_ds;       // [num_tokens] each token's decoder slot (or -1), from K3a for K3b
   float inv127, inv_rk, inv_rv;
 };
+
+// Decoder slot of the request whose first block is blk0, or -1.
+__device__ __forceinline__ int decoder_of_block(const WriteArgs& a, int blk0) {
+  const int ds = blk0 >= 0 && blk0 < a.num_blocks ? a.dec_map[blk0] : -1;
+  return ds < 0 || ds >= a.n_dec_slots ? -1 : ds;
+}
 
 // Request of token i (qsl[r] <= i < qsl[r+1]; qsl is non-decreasing) and its decoder slot, or
 // -1. Decode tokens come first in a step, one per request, so token i is usually request i: that
@@ -94,8 +100,7 @@ __device__ int token_decoder(const WriteArgs& a, int i) {
     const int r = cnt - 1;
     if (r >= 0 && i < a.qsl[r + 1]) blk0 = a.bt[(int64_t)r * a.bt_row_stride];
   }
-  const int ds = blk0 >= 0 && blk0 < a.num_blocks ? a.dec_map[blk0] : -1;
-  return (ds < 0 || ds >= a.n_dec_slots) ? -1 : ds;
+  return decoder_of_block(a, blk0);
 }
 
 // Exact top-k select + quantise + pack of one 128-lane row held as lane l: x0 = dim l,
@@ -235,13 +240,15 @@ __host__ __device__ inline int project_slices(const Geom& g) {
   return (g.r1 + kSliceRanks - 1) / kSliceRanks;
 }
 
-// Chunks of tokens (n_single .. num_tokens) go through the same two launches in tiles of kTok
-// tokens, so that a request's pseudo-inverse and decoder are read once per tile and not once per
-// token, and both contractions run on MFMA.
+// A tile: up to kTok tokens of one request, so that its pseudo-inverse and decoder are read once
+// per tile and not once per token, and both contractions run on MFMA. (Tiles of 16 tokens whatever
+// their requests need a pass per distinct decoder, about 7 us each one after another: 128 requests of 3
+// tokens took 78 us, token by token 44.)
 constexpr int kTok = 16;
 
-__host__ __device__ inline int tile_count(const WriteArgs& a) {
-  return (a.num_tokens - a.n_single + kTok - 1) / kTok;
+// At most so many tiles hold n tokens of num_reqs requests (and those before and after them all).
+__host__ inline int tile_bound(int n, int num_reqs) {
+  return (int)((n + (int64_t)(kTok - 1) * std::min<int64_t>((int64_t)num_reqs + 2, n)) / kTok);
 }
 
 // The tile of block b of a launch's tile part, `per` blocks per tile. Blocks go round-robin over the
@@ -250,29 +257,44 @@ __host__ __device__ inline int tile_count(const WriteArgs& a) {
 __device__ __forceinline__ int tile_of(int b, int per) { return (b >> 3) / per * 8 + (b & 7); }
 __host__ inline int tile_blocks(int tiles, int per) { return (tiles + 7) / 8 * 8 * per; }
 
-// Decoder slot of token i0 + lane (lanes 0 .. n - 1; -1 elsewhere), as token_decoder finds it for
-// one token. Lane j takes request j's span and, in the same round trip, its first block id, then
-// its decoder slot; a ballot per token finds the span it lies in. Every lane must call it.
-__device__ int tile_decoder(const WriteArgs& a, int i0, int n) {
+// The tokens of one tile, tokens il0 .. il0 + nt - 1 of the launch (nt = 0: no such tile), and
+// their request's first block id (-1: none).
+struct TileTokens {
+  int il0, nt, blk0;
+};
+
+// Tiles are numbered request by request; the tokens before the first request and after the last,
+// which are refused unless they are padding, count as requests without a block. Lane j takes span j
+// of 64 (one round trip), a scan of their tile counts finds the tile's. Every lane of the wave must
+// call it; all get the same answer.
+__device__ TileTokens find_tile(const WriteArgs& a, int tile) {
   const int lane = threadIdx.x & 63;
-  int ds = -1;
-  for (int j0 = 0; j0 < a.num_reqs; j0 += 64) {
-    const int j = min(j0 + lane, a.num_reqs - 1);
-    const int lo = a.qsl[j], hi = j0 + lane < a.num_reqs ? a.qsl[j + 1] : lo;
-    const int blk0 = a.bt[(int64_t)j * a.bt_row_stride];
-    int d = -1;
-    if (lo < i0 + n && hi > i0 && blk0 >= 0 && blk0 < a.num_blocks) d = a.dec_map[blk0];
-    if (d >= a.n_dec_slots) d = -1;
+  const int s0 = a.tok0, s1 = a.tok0 + a.num_tokens;
+  int before = 0;
+  for (int j0 = 0; j0 < a.num_reqs + 2; j0 += 64) {  // span j: request j - 1
+    const int j = j0 + lane, r = j - 1;
+    int lo = j > 0 && r <= a.num_reqs ? a.qsl[r] : s0;
+    int hi = j <= a.num_reqs ? a.qsl[j] : s1;
+    const int blk = r >= 0 && r < a.num_reqs ? a.bt[(int64_t)r * a.bt_row_stride] : -1;
+    lo = min(max(lo, s0), s1);
+    hi = min(max(hi, lo), s1);
+    const int own = r <= a.num_reqs ? (hi - lo + kTok - 1) / kTok : 0;
+    int upto = own;
 #pragma unroll
-    for (int t = 0; t < kTok; ++t) {
-      const uint64_t in = __ballot(lo <= i0 + t && i0 + t < hi);
-      if (in) {
-        const int dt = __builtin_amdgcn_readlane(d, __builtin_ctzll(in));
-        ds = lane == t ? dt : ds;
-      }
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(upto, o);
+      upto += lane >= o ? up : 0;
     }
+    const uint64_t in = __ballot(before + upto - own <= tile && tile < before + upto);
+    if (in) {
+      const int l = __builtin_ctzll(in);
+      auto at = [&](int v) { return __builtin_amdgcn_readlane(v, l); };
+      const int first = at(lo) + (tile - (before + at(upto) - at(own))) * kTok;
+      return {first - s0, min(kTok, at(hi) - first), at(blk)};
+    }
+    before += __builtin_amdgcn_readlane(upto, 63);
   }
-  return lane < n && ds >= 0 ? ds : -1;
+  return {0, 0, -1};
 }
 
 __host__ __device__ inline int rank_groups(const Geom& g) { return (g.r1 + 15) / 16; }
@@ -316,9 +338,8 @@ struct RawAct4 {
 // holds dims 4gq .. 4gq + 3 of its token and of its rank (one wide load each), and step j takes
 // element j of both, so the contraction runs in an order of its own but over every dim once.
 // Four accumulators take the steps j = 0..3 and are added pairwise, then the four waves' sums,
-// so no chain of additions is longer than one wave's dims / 16. One pass per distinct decoder
-// among the tile's tokens (one, but where a tile straddles two requests). The keys are requested
-// before the decoders are looked up.
+// so no chain of additions is longer than one wave's dims / 16. The keys are requested before the
+// decoder is looked up.
 // Bound: the round trips of the lookup and of the operands, 64 KB of pinv rows per workgroup from
 // L2. 2,048 tokens: 18.8 us, where a workgroup per (token, 4 ranks) takes 103 us (450 KB of
 // pinv per token).
@@ -328,12 +349,13 @@ __global__ __launch_bounds__(kWThreads) void project_tiles_kernel(WriteArgs a) {
   const Geom& g = a.g;
   const int rgs = rank_groups(g);
   const int tile = tile_of(blockIdx.x, rgs), rg = (int)(blockIdx.x >> 3) % rgs;
-  if (tile >= tile_count(a)) return;
+  if (tile >= a.tiles) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, gq = lane >> 4;
-  const int il0 = a.n_single + tile * kTok;  // first token of the tile in this launch
-  const int nt = min(kTok, a.num_tokens - il0);
+  const TileTokens tt = find_tile(a, tile);
+  if (tt.nt == 0) return;
+  const int il0 = tt.il0, nt = tt.nt;
   const int i0 = a.tok0 + il0;
   const int HD = g.H * kD;
   const int groups = HD >> 6;  // 16-dim groups per wave: 2 H
@@ -347,49 +369,41 @@ __global__ __launch_bounds__(kWThreads) void project_tiles_kernel(WriteArgs a) {
   load_keys(0);
   __builtin_amdgcn_sched_barrier(0);
   const int64_t slot = lane < nt ? a.slot_mapping[i0 + lane] : -1;
-  const int ds = tile_decoder(a, i0, nt);
+  const int ds = decoder_of_block(a, tt.blk0);
   if (rg == 0 && tid < nt) a.ws_ds[il0 + tid] = ds;
-  const uint64_t all = __ballot(ds >= 0 && slot >= 0 && slot < a.n_slots);
+  const uint64_t ok = __ballot(slot >= 0 && slot < a.n_slots);
+  if (ds < 0 || !ok) return;  // alike in every wave; K3b reports it
   const int rank = 16 * rg + n;
-  for (uint64_t todo = all; todo;) {  // wave-uniform, and alike in every wave
-    const int d = __builtin_amdgcn_readlane(ds, __builtin_ctzll(todo));
-    const uint64_t mine = __ballot(ds == d) & todo;
-    if (todo != all) load_keys(0);
-    todo &= ~mine;
-    const float* prow = a.pinv_pool + ((int64_t)d * g.r1 + min(rank, g.r1 - 1)) * HD +
-                        16 * wv * groups + 4 * gq;
-    float4v acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f},
-                      {0.f, 0.f, 0.f, 0.f}};
-    for (int u0 = 0; u0 < groups; u0 += kStep) {
-      float4v pv[kStep];
+  const float* prow = a.pinv_pool + ((int64_t)ds * g.r1 + min(rank, g.r1 - 1)) * HD +
+                      16 * wv * groups + 4 * gq;
+  float4v acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f},
+                    {0.f, 0.f, 0.f, 0.f}};
+  for (int u0 = 0; u0 < groups; u0 += kStep) {
+    float4v pv[kStep];
 #pragma unroll
-      for (int u = 0; u < kStep; ++u)
-        pv[u] = *gbl((const float4v*)(prow + 16 * min(u0 + u, groups - 1)));
-      if (u0) load_keys(u0);
-      // (the scheduler would otherwise spread the loads between the MFMAs and wait for each)
-      __builtin_amdgcn_sched_barrier(0);
+    for (int u = 0; u < kStep; ++u)
+      pv[u] = *gbl((const float4v*)(prow + 16 * min(u0 + u, groups - 1)));
+    if (u0) load_keys(u0);
+    // (the scheduler would otherwise spread the loads between the MFMAs and wait for each)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < kStep; ++u) {
-        const bool in = u0 + u < groups;  // past the last group: zeros
+    for (int u = 0; u < kStep; ++u) {
+      const bool in = u0 + u < groups;  // past the last group: zeros
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kx[u].value(j) : 0.f,
-                                                        in ? pv[u][j] : 0.f, acc[j], 0, 0, 0);
-      }
+      for (int j = 0; j < 4; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kx[u].value(j) : 0.f,
+                                                      in ? pv[u][j] : 0.f, acc[j], 0, 0, 0);
     }
-    const float4v s = (acc[0] + acc[1]) + (acc[2] + acc[3]);  // tokens 4gq .. 4gq + 3, rank n
+  }
+  const float4v s = (acc[0] + acc[1]) + (acc[2] + acc[3]);  // tokens 4gq .. 4gq + 3, rank n
 #pragma unroll
-    for (int i = 0; i < 4; ++i) part[wv][4 * gq + i][n] = s[i];
-    __syncthreads();
-    {
-      const int t = tid >> 4, r = tid & 15;
-      if (((mine >> t) & 1) && 16 * rg + r < g.r1) {
-        const float c = (part[0][t][r] + part[1][t][r]) + (part[2][t][r] + part[3][t][r]);
-        a.ws_c[(int64_t)(il0 + t) * g.r1 + 16 * rg + r] = c;
-        if (a.c_out) a.c_out[(int64_t)(i0 + t) * g.r1 + 16 * rg + r] = c;
-      }
-    }
-    __syncthreads();
+  for (int i = 0; i < 4; ++i) part[wv][4 * gq + i][n] = s[i];
+  __syncthreads();
+  const int t = tid >> 4, r = tid & 15;
+  if (((ok >> t) & 1) && 16 * rg + r < g.r1) {
+    const float c = (part[0][t][r] + part[1][t][r]) + (part[2][t][r] + part[3][t][r]);
+    a.ws_c[(int64_t)(il0 + t) * g.r1 + 16 * rg + r] = c;
+    if (a.c_out) a.c_out[(int64_t)(i0 + t) * g.r1 + 16 * rg + r] = c;
   }
 }
 
@@ -501,19 +515,19 @@ __global__ __launch_bounds__(kPThreads, 6) void pack_tiles_kernel(WriteArgs a) {
   __shared__ __align__(16) PackTileSmem S;
   const Geom& g = a.g;
   const int tile = tile_of(blockIdx.x, g.H), h = (int)(blockIdx.x >> 3) % g.H;
-  if (tile >= tile_count(a)) return;
+  if (tile >= a.tiles) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, gq = lane >> 4;
-  const int il0 = a.n_single + tile * kTok;
-  const int nt = min(kTok, a.num_tokens - il0);
+  const TileTokens tt = find_tile(a, tile);
+  if (tt.nt == 0) return;
+  const int il0 = tt.il0, nt = tt.nt;
   const int i0 = a.tok0 + il0;
   const int HD = g.H * kD;
   const int R = dec_ranks(g.r1);
-  // the tile's slots and decoders (lane t: token t), and this wave's tokens' rows
+  // the tile's slots (lane t: token t) and decoder, and this wave's tokens' rows
   const int64_t slot = lane < nt ? a.slot_mapping[i0 + lane] : -1;
-  int ds = -1;
-  if (!a.cq_in && lane < nt) ds = a.ws_ds[il0 + lane];
+  const int ds = a.cq_in ? decoder_of_block(a, tt.blk0) : a.ws_ds[il0];
   // (every load unconditional and behind no branch of its own, so that all are in flight together)
   const int nk = R >> 6;  // 64-rank groups in use
   float xk[kPTok][2], xv[kPTok][2], cw[kPTok][4] = {}, csin[kPTok];
@@ -550,7 +564,6 @@ __global__ __launch_bounds__(kPThreads, 6) void pack_tiles_kernel(WriteArgs a) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) cw[t][k] = lane + 64 * k < g.r1 ? cw[t][k] : 0.f;
   }
-  if (a.cq_in) ds = tile_decoder(a, i0, nt);
   const bool live = slot >= 0;  // a negative slot id is vLLM's PAD_SLOT_ID: skipped silently
   if (h == 0 && wv == 0) {
     const bool bad_slot = __ballot(live && slot >= a.n_slots) != 0;
@@ -643,16 +656,13 @@ __global__ __launch_bounds__(kPThreads, 6) void pack_tiles_kernel(WriteArgs a) {
   }
   __syncthreads();
   // ---- the decoder's part of the keys: rec[token][dim], dims 16w .. 16w + 15 in this wave
-  float4v rec = {0.f, 0.f, 0.f, 0.f};  // dims 16w + 4gq .. + 3 of token n
-  const int ds_n = __shfl(ds, n);
-  for (uint64_t todo = ok; todo;) {  // one pass per distinct decoder, alike in every wave
-    const int d = __builtin_amdgcn_readlane(ds, __builtin_ctzll(todo));
-    todo &= ~__ballot(ds == d);
+  float4v rec;  // dims 16w + 4gq .. + 3 of token n
+  {
     // per 64 ranks lane (n, gq) holds ranks 16gq .. 16gq + 15 of dim n (one 16-byte load) and of
     // token n; MFMA step (c, j) takes rank 16gq + 4c + j of every lane group
     float4v acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    const float* decs = a.dec_scale + (int64_t)d * R + 16 * gq;
-    const int8_t* decq = a.dec_q + ((int64_t)d * HD + h * kD + 16 * wv + n) * R + 16 * gq;
+    const float* decs = a.dec_scale + (int64_t)ds * R + 16 * gq;
+    const int8_t* decq = a.dec_q + ((int64_t)ds * HD + h * kD + 16 * wv + n) * R + 16 * gq;
     for (int s = 0; s < R; s += 64) {
       const u32x4 q16 = *gbl((const u32x4*)(decq + s));
       float4v rul[4];
@@ -671,8 +681,7 @@ __global__ __launch_bounds__(kPThreads, 6) void pack_tiles_kernel(WriteArgs a) {
           acc[c & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], cq[j], acc[c & 1], 0, 0, 0);
       }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rec[i] = ds_n == d ? acc[0][i] + acc[1][i] : rec[i];
+    rec = acc[0] + acc[1];
   }
   *(float4v*)&S.rec[n][16 * wv + 4 * gq] = rec;
   __syncthreads();
@@ -872,10 +881,12 @@ static void launch_project_tiles(const WriteArgs& b, int grid, hipStream_t st) {
   hipLaunchKernelGGL(kfn, dim3(grid), dim3(kWThreads), 0, st, b);
 }
 
-// Fewest chunk tokens that go in tiles: below, the tiles' few workgroups leave most of the chip
-// idle. One request, per call: 128 tokens 19.4 us singly and 21.1 in tiles, 256 tokens 23.7 and
-// 21.4, 1,024 tokens 70 and 30.
-constexpr int kMinTiled = 192;
+// Fewest tokens of a launch that go in tiles: kMinTiled, and kTiledPerReq more for every further
+// request (each can leave a tile partly filled, down to one token). Single tokens against tiles, graph
+// replays, us: one request of 192 tokens 21.4 / 21.8, of 208 22.3 / 21.8, of 1,024 73.8 / 29.3; 2 x 97
+// 21.2 / 21.1, 8 x 64 42.3 / 21.4, 64 x 4 30.0 / 26.6, 128 x 3 44.6 / 41.5, 256 x 3 83.2 / 76.7, 256 x 2
+// 64.1 / 73.9; one token each of 31 requests and 200 of another 25.1 / 26.6, of 255 and 465 78.2 / 81.4.
+constexpr int kMinTiled = 208, kTiledPerReq = 3;
 
 static float inv_ruler_f32(int bits) { return (float)(1.0 / (double)((1 << (bits - 1)) - 1)); }
 
@@ -961,28 +972,26 @@ int write_paged(const Geom& g, const void* key, int k_dtype, int64_t k_row_strid
       b.ws_c = (float*)((char*)ws + kCounterBytes);
       b.ws_ds = (int*)(b.ws_c + (int64_t)b.num_tokens * g.r1);
     }
-    // One token per request is the decode step's write: token by token, spread over the chip. A
-    // step's decode tokens lie among its first num_reqs; what follows is chunks, in tiles.
-    b.n_single = num_reqs > 1 ? std::min(std::max(num_reqs - t0, 0), b.num_tokens) : 0;
-    if (b.num_tokens - b.n_single < kMinTiled) b.n_single = b.num_tokens;
-    const int tiles = tile_count(b);
-    if (!cq_in) {
-      if (b.n_single)
-        hipLaunchKernelGGL(write_project_kernel, dim3(b.n_single * project_slices(g)),
-                           dim3(kWThreads), 0, st, b);
-      const int grid = tile_blocks(tiles, rank_groups(g));
-      if (tiles && k_dtype == TTKV_DTYPE_F32) launch_project_tiles<TTKV_DTYPE_F32>(b, grid, st);
-      if (tiles && k_dtype == TTKV_DTYPE_F16) launch_project_tiles<TTKV_DTYPE_F16>(b, grid, st);
-      if (tiles && k_dtype == TTKV_DTYPE_BF16) launch_project_tiles<TTKV_DTYPE_BF16>(b, grid, st);
-    }
+    b.tiles = tile_bound(b.num_tokens, num_reqs);
+    const bool tiled = b.num_tokens >= kMinTiled + (int64_t)kTiledPerReq * std::max(num_reqs - 1, 0);
     const bool b3 = g.res_bits == 3;
-    if (b.n_single) {
+    if (!tiled) {
+      if (!cq_in)
+        hipLaunchKernelGGL(write_project_kernel, dim3(b.num_tokens * project_slices(g)),
+                           dim3(kWThreads), 0, st, b);
       auto kfn = b3 ? write_pack_kernel<3, 3> : write_pack_kernel<4, 4>;
-      hipLaunchKernelGGL(kfn, dim3(b.n_single * g.H), dim3(kWThreads), 0, st, b);
+      hipLaunchKernelGGL(kfn, dim3(b.num_tokens * g.H), dim3(kWThreads), 0, st, b);
+      continue;
     }
-    const int grid = tile_blocks(tiles, g.H);
-    if (tiles && b3) launch_pack_tiles<3, 3>(b, grid, st);
-    if (tiles && !b3) launch_pack_tiles<4, 4>(b, grid, st);
+    if (!cq_in) {
+      const int grid = tile_blocks(b.tiles, rank_groups(g));
+      if (k_dtype == TTKV_DTYPE_F32) launch_project_tiles<TTKV_DTYPE_F32>(b, grid, st);
+      if (k_dtype == TTKV_DTYPE_F16) launch_project_tiles<TTKV_DTYPE_F16>(b, grid, st);
+      if (k_dtype == TTKV_DTYPE_BF16) launch_project_tiles<TTKV_DTYPE_BF16>(b, grid, st);
+    }
+    const int grid = tile_blocks(b.tiles, g.H);
+    if (b3) launch_pack_tiles<3, 3>(b, grid, st);
+    if (!b3) launch_pack_tiles<4, 4>(b, grid, st);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return host_fail(TTKV_E_LAUNCH, std::string("write launch: ") +
