@@ -363,3 +363,26 @@ def test_serving_limits_from_a_config_loaded_later(monkeypatch):
     monkeypatch.setitem(__import__("sys").modules, "vllm.config",
                         SimpleNamespace(get_current_vllm_config=lambda: vc))
     assert impl.serving_limits(1234) == (31, 99)
+
+
+def test_serving_limits_from_a_vllm_that_can_be_imported_later(monkeypatch, tmp_path):
+    """A call that found no vllm does not hide one that is put on the path after it."""
+    import importlib
+    import sys
+    monkeypatch.delenv("VLLM_TTKV_MAX_NUM_SEQS", raising=False)
+    monkeypatch.delenv("VLLM_TTKV_MAX_MODEL_LEN", raising=False)
+    assert impl.serving_limits(1234) == (256, 1234)
+    pkg = tmp_path / "vllm"
+    pkg.mkdir()
+    (pkg / "__init__.py").write_text("")
+    (pkg / "config.py").write_text(
+        "from types import SimpleNamespace as N\n"
+        "def get_current_vllm_config():\n"
+        "    return N(scheduler_config=N(max_num_seqs=7), model_config=N(max_model_len=55))\n")
+    monkeypatch.syspath_prepend(str(tmp_path))
+    importlib.invalidate_caches()
+    try:
+        assert impl.serving_limits(1234) == (7, 55)
+    finally:
+        for name in ("vllm.config", "vllm"):
+            sys.modules.pop(name, None)

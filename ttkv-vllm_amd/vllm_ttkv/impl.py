@@ -35,7 +35,6 @@ from __future__ import annotations
 
 import logging
 import os
-import sys
 from dataclasses import dataclass
 
 import torch
@@ -44,7 +43,7 @@ from . import _hip, kernels
 from . import encode as enc
 from .layout import TTKLayout, config_named
 from .patch import take_raw_k
-from .rope_store import decoder_for_layer, ensure_store, layout_for_layer
+from .rope_store import decoder_for_layer, ensure_store, layout_for_layer, store_for_layer
 
 logger = logging.getLogger("vllm.ttkv")
 
@@ -61,27 +60,18 @@ MAX_LEN_ENV = "VLLM_TTKV_MAX_MODEL_LEN"
 DEFAULT_MAX_SEQS = 256
 
 
-_NO_VLLM = False
-
-
 def serving_limits(fallback_len: int | None = None) -> tuple[int, int | None]:
     """(max_num_seqs, max_model_len) the fixed buffers are sized for: the environment
     (`VLLM_TTKV_MAX_NUM_SEQS`, `VLLM_TTKV_MAX_MODEL_LEN`) over the running vLLM config, else 256
     sequences and `fallback_len` (the RoPE table's length: no position beyond it has an angle)."""
-    global _NO_VLLM
     seqs = lens = None
-    if not _NO_VLLM or "vllm" in sys.modules or "vllm.config" in sys.modules:
-        try:
-            from vllm.config import get_current_vllm_config
-            vc = get_current_vllm_config()
-            seqs = getattr(getattr(vc, "scheduler_config", None), "max_num_seqs", None)
-            lens = getattr(getattr(vc, "model_config", None), "max_model_len", None)
-        except ModuleNotFoundError as e:
-            # every layer of every step asks: a package that is not installed is searched for
-            # once, and found again as soon as a module of that name is loaded
-            _NO_VLLM = (e.name or "").split(".")[0] == "vllm" and "vllm" not in sys.modules
-        except Exception:  # noqa: BLE001
-            pass
+    try:
+        from vllm.config import get_current_vllm_config
+        vc = get_current_vllm_config()
+        seqs = getattr(getattr(vc, "scheduler_config", None), "max_num_seqs", None)
+        lens = getattr(getattr(vc, "model_config", None), "max_model_len", None)
+    except Exception:  # noqa: BLE001
+        pass
     seqs = int(os.environ.get(MAX_SEQS_ENV) or seqs or DEFAULT_MAX_SEQS)
     lens = os.environ.get(MAX_LEN_ENV) or lens or fallback_len
     return seqs, (None if lens is None else int(lens))
@@ -254,9 +244,11 @@ class TTKVAttentionImpl(_ImplBase):
         name = getattr(layer, "layer_name", None)
         stash = take_raw_k(name)                # pops: the write comes first, unconditionally
         csc = self._cos_sin_cache(layer, stash)
-        self._limits = serving_limits(int(csc.shape[0]))
+        self._table_len = int(csc.shape[0])
+        new = store_for_layer(name) is None
         store = ensure_store(name, csc, self.num_heads, self.num_kv_heads, self.head_size, lay,
-                             num_blocks=int(cache.shape[0]), capacity=self._limits[0])
+                             num_blocks=int(cache.shape[0]),
+                             capacity=self._limits()[0] if new else None)
         self._write_store(lay, cache, stash, value, md, plan, store)
 
         q3 = query.view(n_tokens, self.num_heads, self.head_size)
@@ -368,14 +360,19 @@ class TTKVAttentionImpl(_ImplBase):
                     for r, c in enumerate(ncomp[:plan.n_reqs].tolist())]
         return [int(x) for x in md.seq_lens[:plan.n_reqs].tolist()]
 
+    def _limits(self):
+        """The serving limits, looked up where a store or a workspace is made and not on every step:
+        an attempt to import a vllm that is not installed takes longer than a kernel launch."""
+        return serving_limits(self._table_len)
+
     def _workspace(self, lay, num_reqs, max_seq_len, block_size, device):
         L = _hip.lib()
         g = _hip.Layout.of(lay)
         need = L.ttkv_decode_workspace_bytes(g, self.num_heads, num_reqs, max_seq_len, block_size)
-        seqs, lens = self._limits
         buf = workspaces(device).bufs.get("decode")
         if buf is not None and buf.numel() >= need:
             return buf
+        seqs, lens = self._limits()
         cap = L.ttkv_decode_workspace_bytes(g, self.num_heads, max(seqs, num_reqs),
                                             max(lens or 0, max_seq_len), block_size)
         return workspaces(device).get("decode", need, cap, fixed=True)
@@ -388,7 +385,7 @@ class TTKVAttentionImpl(_ImplBase):
             buf = workspaces(device).bufs.get("decode_write")
             if buf is not None and buf.numel() >= need:
                 return buf
-            cap = L.ttkv_write_workspace_bytes(g, max(self._limits[0], num_tokens))
+            cap = L.ttkv_write_workspace_bytes(g, max(self._limits()[0], num_tokens))
             return workspaces(device).get("decode_write", need, cap, fixed=True)
         return workspaces(device).get("prefill_write", need)
 
