@@ -4,13 +4,33 @@ request, whole ones and the head of another. Against the CPU oracle, request by 
 import pytest
 import torch
 
-from helpers import dec_pool_of, fitted_store, llama3_cache, paged
+from helpers import dec_pool_of, device_store, fitted_store, llama3_cache, paged
 from oracle import attend
 from vllm_ttkv import kernels, synth
 
 pytestmark = pytest.mark.gpu
 MAX_ABS, MEAN_ABS = 2e-3, 1e-3
 SCALE = 128 ** -0.5
+
+
+def _takes_ranges(lens, H, block_size=16):
+    """Whether the device's plan cuts this batch into ranges (the rule of the kernel's work plan)."""
+    def up(a, b):
+        return -(-a // b)
+    target = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    tiles = [max(1, up(n, 64)) for n in lens]
+    cap = max(min(258 * block_size // 64, 64), 1)
+
+    def items(m):
+        return H * sum(max(1, up(up(n, 64), m)) for n in lens)
+    rounds = max(1, up(len(lens) * H, target))
+    m = next((m for m in range(1, cap) if items(m) <= rounds * target), cap)
+    teams = max(1, target // H)
+    units = sum(tiles) + len(lens)
+    share = up(units, teams)
+    longest = max(min(t, m) for t in tiles)
+    return (len(lens) > 1 and units > 2 * teams and share < cap
+            and 16 * up(items(m), target) * (longest + 1) > 18 * (share + 1))
 
 
 def _batch(cfg, lens, H, G, r1, seed, dtype, empty=(), lost=(), block_size=16, workspace=None):
@@ -63,6 +83,7 @@ RAGGED = [1500, 1, 17, 64, 65, 130, 257, 900]
 def test_ragged_requests_in_ranges(cfg, H, G, r1, dtype):
     print(f"[k1 ranges] {cfg} H={H} G={G} r1={r1} {dtype}", flush=True)
     lens = RAGGED * (8 if H == 8 else 20)
+    assert _takes_ranges(lens, H)
     _batch(cfg, lens, H, G, r1, seed=5, dtype=dtype)
 
 
@@ -70,6 +91,7 @@ def test_empty_and_undecodable_requests_in_ranges():
     """Empty contexts give zeros and requests without a decoder NaN (error bit 1), at the head of
     a range, in its middle and in a row; the others are unaffected."""
     lens = RAGGED * 9
+    assert _takes_ranges(lens, 8)
     got = _batch("safe", lens, 8, 3, 110, seed=6, dtype=torch.float16,
                  empty=(0, 1, 2, 20, 33, 34, 71), lost=(3, 8, 21, 40, 41, 63))
     assert got.shape[0] == 72
@@ -79,6 +101,7 @@ def test_one_workspace_for_ranges_and_chunks():
     """A range batch, a uniform one and the range batch again on one workspace: the counters come
     back to zero and the repeat is bit-identical."""
     lens = RAGGED * 9
+    assert _takes_ranges(lens, 8) and not _takes_ranges([900] * 5, 8)
     lay = fitted_store("safe", 64, seed=5 + 64)["lay"]
     need = kernels.decode_workspace(lay, 24, len(lens), max(lens), "cuda").numel()
     ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
@@ -87,3 +110,38 @@ def test_one_workspace_for_ranges_and_chunks():
     b = _batch("safe", lens, 8, 3, 110, seed=7, dtype=torch.float16, workspace=ws)
     assert torch.equal(a, b)
     assert int(ws[:65536].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("cfg,block_size,where,dtype", [
+    ("safe", 16, 63, torch.float16), ("safe", 32, 0, torch.bfloat16),
+    ("campaign4x", 64, 31, torch.float16), ("safe_fp16", 16, 40, torch.float16),
+    ("campaign4x_int4g32", 32, 5, torch.bfloat16)])
+def test_a_long_request_among_short_ones(cfg, block_size, where, dtype):
+    """One request in more partials than a thread's registers combine: the workgroup that combines
+    them weighs them in the tile buffers, and opens its next segment there."""
+    print(f"[k1 ranges] {cfg} block {block_size} long at {where} {dtype}", flush=True)
+    lens = [70 + 3 * i for i in range(63)]
+    lens.insert(where, 14000)
+    assert _takes_ranges(lens, 8, block_size)
+    st = device_store(cfg, lens, seed=8, block_size=block_size)
+    q = synth.queries(64, HQ=24, seed=12, dtype=dtype)
+    cache = llama3_cache(16384)
+    dev = "cuda"
+    out = torch.full((64, 24, 128), float("nan"), dtype=dtype, device=dev)
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    args = (st["play"], q.to(dev), st["page"], block_size, st["block_table"], st["seq_lens"],
+            torch.arange(65, dtype=torch.int32, device=dev), 14000, st["dec_map"],
+            st["dec_pool"], cache.to(dev), SCALE)
+    ws = kernels.decode_workspace(st["play"], 24, 64, 14000, dev, block_size)
+    kernels.decode_paged(*args, out=out, error_word=err, workspace=ws)
+    got = out.float().cpu()
+    kernels.decode_paged(*args, out=out.fill_(0), error_word=err, workspace=ws)
+    assert torch.equal(out.float().cpu(), got) and int(err.item()) == 0
+    page, bt = st["page"].cpu(), st["block_table"].cpu()
+    tol = 1.0 if dtype == torch.float16 else 8.0
+    for r in range(64):
+        want = attend.paged_decode(st["lay"], page, bt[r:r + 1], torch.tensor([lens[r]]),
+                                   torch.arange(2), q[r:r + 1].float(), [st["decoders"][r]],
+                                   cache, block_size, SCALE, dtype=torch.float64)
+        e = (got[r].double() - want[0]).abs()
+        assert e.max() <= tol * MAX_ABS and e.mean() <= tol * MEAN_ABS, (r, lens[r], e.max())
