@@ -17,14 +17,18 @@
 //                  vrul     [64] fp32               -- the V row rulers
 //                Keys past the context are written as zeros (masked by the causal rule).
 //   K2b attend : flash attention over those tiles. A 512-thread workgroup owns 128 queries x G
-//                heads of one (request, KV head, key split); wave w owns queries 16w..16w+15.
+//                heads of one (request, KV head, key split), wave w queries 16w..16w+15 of every
+//                head; at G = 4 96 queries x 4 heads, their 24 groups of (head, 16 queries) three
+//                to a wave. Launches whose longest chunk is at most half of that (PAIR) lay the
+//                rows over waves 0..3, and waves 4..7 take the second half of every tile's keys
+//                for the same rows.
 //                Per 64-key tile: S^T = K Q^T on MFMA (hi and lo key halves against the fp16
 //                query), causal -inf, online base-2 softmax per query column, O^T += Vt (P *
 //                ruler_v)^T on MFMA with P * ruler_v * 2^-ve rounded to fp16 once (ve >= 0 grows
 //                with the largest V ruler seen, keeping it below 2^15), in 32-key halves.
-//                Waves 4..7 run half a tile behind waves 0..3 (three LDS tile buffers, one
-//                barrier per tile), so each SIMD's two waves overlap MFMA with softmax. The
-//                next tile is copied to LDS while the current ones are
+//                Without PAIR, waves 4..7 run half a tile behind waves 0..3 (three LDS tile
+//                buffers, one barrier per tile), so each SIMD's two waves overlap MFMA with
+//                softmax. The next tile is copied to LDS while the current ones are
 //                computed, by direct global -> LDS DMA issued at the barrier. Key splits are
 //                combined in the same launch by the last workgroup.
 //
@@ -650,11 +654,12 @@ __global__ __launch_bounds__(kAThreads, 2) void attend_kernel(AttendArgs a) {
     }
   };
 
-  // Waves 4..7 run half a tile behind waves 0..3, so that the two waves sharing a SIMD are in
-  // different phases (one's MFMAs beside the other's softmax). Barrier k: waves 0..3 have
+  // Without PAIR, waves 4..7 run half a tile behind waves 0..3, so that the two waves sharing a SIMD
+  // are in different phases (one's MFMAs beside the other's softmax). Barrier k: waves 0..3 have
   // finished tiles < k, waves 4..7 tiles < k - 1 and half 0 of tile k - 1. Between barriers k
   // and k + 1 tiles k - 1 and k are read and tile k + 1 is written, into buffer (k + 1) % 3,
-  // whose last reader (tile k - 2) finished before barrier k.
+  // whose last reader (tile k - 2) finished before barrier k. (PAIR: every wave is done with tile k
+  // before barrier k + 1.)
   dma_tile(S.t[0], tl0);
   const bool late = wv >= 4;
   for (int k = 0; k <= ntl_item; ++k) {

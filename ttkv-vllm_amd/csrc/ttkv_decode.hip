@@ -3,9 +3,11 @@
 //
 // Work item = (request r, KV head h, token chunk c). The chunk length comes from the batch's own
 // lengths, computed on the device by every workgroup (the work plan below), so a ragged batch
-// spreads its total tokens over one round of resident workgroups. A 256-thread workgroup (4
-// waves) walks its chunk in 64-token tiles with the next tile's raw bytes prefetched into
-// registers while the current one is computed:
+// spreads its total tokens over one round of resident workgroups. Where such chunks leave the chip
+// uneven, the tiles of all requests are cut into equal ranges instead, and a workgroup walks its
+// range as several segments, one per request. A 256-thread workgroup (4 waves) walks a chunk or
+// segment in 64-token tiles with the next tile's raw bytes prefetched into registers while the
+// current one is computed:
 //   commit  : prefetched bytes -> LDS: coefficients as fp16 MFMA B-fragments (int8 is exact in
 //             fp16; the fp16 mode's values are copied; the 4-bit mode's q * group scale is exact
 //             in fp16, commit_coef); this head's K and V rows realigned, the code streams
@@ -36,7 +38,7 @@
 //             ruler seen, so P' stays below 2^15) and the codes as exact fp16 integers
 //             (c - 2^(b-1)). The V^T operand is read straight from the decoded code rows with
 //             the gfx950 LDS transpose read (ds_read_tr8_b64); P'^T from a per-wave LDS row.
-// Chunks of one (r, h) are combined in the same launch by the last workgroup to finish
+// Chunks (segments) of one (r, h) are combined in the same launch by the last workgroup to finish
 // (write-through partials + a relaxed arrival counter, agent-scope loads), which also resets the
 // counter to zero. The counters sit at the
 // workspace's fixed 64 KiB head, the partials after it, indexed by (chunk item) so their count
@@ -476,616 +478,619 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
   auto finish = [&](const auto& a, Smem& S, int tid, int h, int r, int c, int n_chunks, int base,
                     int64_t qrow, float4v (&oacc)[2], float (&m_run)[G], float (&l_lane)[G],
                     int ve) __attribute__((always_inline)) {
-  const auto& g = a.g;
-  const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
-  const int dl = 16 * wv + 4 * gq;
-  // the V-ruler scale 2^-ve taken back (exact)
-  if (ve != 0) {
-    const float vsc = ldexpf(1.f, ve);
+    const auto& g = a.g;
+    const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
+    const int dl = 16 * wv + 4 * gq;
+    // the V-ruler scale 2^-ve taken back (exact)
+    if (ve != 0) {
+      const float vsc = ldexpf(1.f, ve);
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi) oacc[mi] *= vsc;
-  }
-  // ---- normalisers: the per-lane partial sums over the wave (every wave holds the same)
-#pragma unroll
-  for (int p = 0; p < G; ++p) l_lane[p] = wave_sum(l_lane[p]);
-  if (tid == 0) {
-#pragma unroll
-    for (int p = 0; p < G; ++p) {
-      S.m[p] = m_run[p];
-      S.l[p] = l_lane[p];
+      for (int mi = 0; mi < 2; ++mi) oacc[mi] *= vsc;
     }
-  }
-  __syncthreads();
+    // ---- normalisers: the per-lane partial sums over the wave (every wave holds the same)
+#pragma unroll
+    for (int p = 0; p < G; ++p) l_lane[p] = wave_sum(l_lane[p]);
+    if (tid == 0) {
+#pragma unroll
+      for (int p = 0; p < G; ++p) {
+        S.m[p] = m_run[p];
+        S.l[p] = l_lane[p];
+      }
+    }
+    __syncthreads();
 
-  if (n_chunks == 1) {
+    if (n_chunks == 1) {
+      if (n < G) {
+        const float inv = 1.f / S.l[n];
+        const int64_t ob = qrow * a.out_row_stride + (int64_t)(h * G + n) * kD;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          store_act(a.out, a.out_dtype, ob + dl + i, oacc[0][i] * inv);
+          store_act(a.out, a.out_dtype, ob + 64 + dl + i, oacc[1][i] * inv);
+        }
+      }
+      return;
+    }
+
+    // ---- split-K partial: [G][kD + 2] per (r, h, c): unnormalised o, running max, running sum
+    const int64_t pstride = (int64_t)G * (kD + 2);
+    float* partp = a.ws_part + ((int64_t)(base + c) * g.H + h) * pstride;
+    // The partial is written with agent-scope (write-through) atomic stores and waited on before
+    // the counter update, so no cache-wide release fence is needed.
+    auto st_agent = [](float* p, float v) {
+      __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     if (n < G) {
-      const float inv = 1.f / S.l[n];
-      const int64_t ob = qrow * a.out_row_stride + (int64_t)(h * G + n) * kD;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        store_act(a.out, a.out_dtype, ob + dl + i, oacc[0][i] * inv);
-        store_act(a.out, a.out_dtype, ob + 64 + dl + i, oacc[1][i] * inv);
+        st_agent(&partp[n * (kD + 2) + dl + i], oacc[0][i]);
+        st_agent(&partp[n * (kD + 2) + 64 + dl + i], oacc[1][i]);
       }
     }
-    return;
-  }
-
-  // ---- split-K partial: [G][kD + 2] per (r, h, c): unnormalised o, running max, running sum
-  const int64_t pstride = (int64_t)G * (kD + 2);
-  float* partp = a.ws_part + ((int64_t)(base + c) * g.H + h) * pstride;
-  // The partial is written with agent-scope (write-through) atomic stores and waited on before
-  // the counter update, so no cache-wide release fence is needed.
-  auto st_agent = [](float* p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  if (n < G) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      st_agent(&partp[n * (kD + 2) + dl + i], oacc[0][i]);
-      st_agent(&partp[n * (kD + 2) + 64 + dl + i], oacc[1][i]);
+    if (tid < G) {
+      st_agent(&partp[tid * (kD + 2) + kD], S.m[tid]);
+      st_agent(&partp[tid * (kD + 2) + kD + 1], S.l[tid]);
     }
-  }
-  if (tid < G) {
-    st_agent(&partp[tid * (kD + 2) + kD], S.m[tid]);
-    st_agent(&partp[tid * (kD + 2) + kD + 1], S.l[tid]);
-  }
-  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    const int prev = arrive(&a.ws_cnt[r * g.H + h]);
-    S.is_last = (prev == n_chunks - 1);
-  }
-  __syncthreads();
-  if (!S.is_last) return;
-  // Every partial was stored write-through and completed before its counter update, so the
-  // agent-scope loads below (ld_agent: coherent across the XCDs' L2s, with no L2 invalidate) see
-  // them; the loads of all chunks are in flight together.
-
-  const float* pbase = a.ws_part + ((int64_t)base * g.H + h) * pstride;
-  const int64_t cstride = (int64_t)g.H * pstride;  // between chunks of one request and head
-  // Many chunks: weights in LDS (the tile buffers are free now) -- every chunk's (max, sum) in
-  // one round of loads, the per-head max and normaliser by one wave per head, then each output's
-  // chunk loads issued together: a few memory round trips whatever the chunk count. Up to 8
-  // chunks (24 for G <= 4), every value a thread's outputs need is requested in one round and
-  // combined in registers (combine_regs): one round trip. (Partials live past this XCD's L2; a round trip took ~2.8 us at
-  // the headline, and the former two rounds per output, four per thread, made this combine
-  // ~11.5 us of the launch's tail.)
-  float* wsh = reinterpret_cast<float*>(&S.coef[0][0]);
-  constexpr int kWCap = (int)(sizeof(S.coef) / sizeof(float));
-  const int ncp = n_chunks * G;
-  const int64_t orow = qrow * a.out_row_stride;
-  if (n_chunks <= 8) {
-    combine_regs<G, 8>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
-  } else if (G <= 4 && n_chunks <= 24) {
-    // (batch 1 at ~1k tokens: 17 chunks per head)
-    if constexpr (G <= 4) combine_regs<G, 24>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
-  } else if (2 * ncp <= kWCap) {
-    for (int i = tid; i < ncp; i += kThreads) {
-      const int cc = i / G, p = i - cc * G;
-      const float* pc = pbase + cc * cstride + p * (kD + 2);
-      wsh[i] = ld_agent(&pc[kD]);
-      wsh[ncp + i] = ld_agent(&pc[kD + 1]);
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const int prev = arrive(&a.ws_cnt[r * g.H + h]);
+      S.is_last = (prev == n_chunks - 1);
     }
     __syncthreads();
-    for (int p = wv; p < G; p += kWaves) {  // wave-uniform: whole waves take a head each
-      float mx = -INFINITY;
-      for (int cc = lane; cc < n_chunks; cc += 64) mx = fmaxf(mx, wsh[cc * G + p]);
-      mx = wave_max(mx);
-      float L = 0.f;
-      for (int cc = lane; cc < n_chunks; cc += 64)
-        L = fmaf(wsh[ncp + cc * G + p], exp2f(wsh[cc * G + p] - mx), L);
-      const float invL = 1.f / wave_sum(L);
-      for (int cc = lane; cc < n_chunks; cc += 64)
-        wsh[cc * G + p] = exp2f(wsh[cc * G + p] - mx) * invL;
-    }
-    __syncthreads();
-    for (int it = tid; it < G * kD; it += kThreads) {
-      const int p = it / kD;
-      const int dim = it - p * kD;
-      const float* po = pbase + p * (kD + 2) + dim;
-      float O = 0.f;
-      for (int c0 = 0; c0 < n_chunks; c0 += 32) {
-        float v[32];
-#pragma unroll
-        for (int j = 0; j < 32; ++j) v[j] = c0 + j < n_chunks ? ld_agent(&po[(c0 + j) * cstride]) : 0.f;
-#pragma unroll
-        for (int j = 0; j < 32; ++j)
-          if (c0 + j < n_chunks) O = fmaf(v[j], wsh[(c0 + j) * G + p], O);
-      }
-      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim, O);
-    }
-  } else {  // more chunks than the LDS weights hold: two passes per output
-    for (int it = tid; it < G * kD; it += kThreads) {
-      const int p = it / kD;
-      const int dim = it - p * kD;
-      float M = -INFINITY;
-#pragma unroll 8
-      for (int cc = 0; cc < n_chunks; ++cc) M = fmaxf(M, ld_agent(&pbase[cc * cstride + p * (kD + 2) + kD]));
-      float L = 0.f, O = 0.f;
-#pragma unroll 8
-      for (int cc = 0; cc < n_chunks; ++cc) {
+    if (!S.is_last) return;
+    // Every partial was stored write-through and completed before its counter update, so the
+    // agent-scope loads below (ld_agent: coherent across the XCDs' L2s, with no L2 invalidate) see
+    // them; the loads of all chunks are in flight together.
+
+    const float* pbase = a.ws_part + ((int64_t)base * g.H + h) * pstride;
+    const int64_t cstride = (int64_t)g.H * pstride;  // between chunks of one request and head
+    // Many chunks: weights in LDS (the tile buffers are free now) -- every chunk's (max, sum) in
+    // one round of loads, the per-head max and normaliser by one wave per head, then each output's
+    // chunk loads issued together: a few memory round trips whatever the chunk count. Up to 8
+    // chunks (24 for G <= 4), every value a thread's outputs need is requested in one round and
+    // combined in registers (combine_regs): one round trip. (Partials live past this XCD's L2; a
+    // round trip took ~2.8 us at the headline, and the former two rounds per output, four per
+    // thread, made this combine ~11.5 us of the launch's tail.)
+    float* wsh = reinterpret_cast<float*>(&S.coef[0][0]);
+    constexpr int kWCap = (int)(sizeof(S.coef) / sizeof(float));
+    const int ncp = n_chunks * G;
+    const int64_t orow = qrow * a.out_row_stride;
+    if (n_chunks <= 8) {
+      combine_regs<G, 8>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
+    } else if (G <= 4 && n_chunks <= 24) {
+      // (batch 1 at ~1k tokens: 17 chunks per head)
+      if constexpr (G <= 4)
+        combine_regs<G, 24>(pbase, cstride, n_chunks, tid, a.out, a.out_dtype, orow, h);
+    } else if (2 * ncp <= kWCap) {
+      for (int i = tid; i < ncp; i += kThreads) {
+        const int cc = i / G, p = i - cc * G;
         const float* pc = pbase + cc * cstride + p * (kD + 2);
-        const float f = exp2f(ld_agent(&pc[kD]) - M);
-        L = fmaf(ld_agent(&pc[kD + 1]), f, L);
-        O = fmaf(ld_agent(&pc[dim]), f, O);
+        wsh[i] = ld_agent(&pc[kD]);
+        wsh[ncp + i] = ld_agent(&pc[kD + 1]);
       }
-      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim,
-                O / L);
+      __syncthreads();
+      for (int p = wv; p < G; p += kWaves) {  // wave-uniform: whole waves take a head each
+        float mx = -INFINITY;
+        for (int cc = lane; cc < n_chunks; cc += 64) mx = fmaxf(mx, wsh[cc * G + p]);
+        mx = wave_max(mx);
+        float L = 0.f;
+        for (int cc = lane; cc < n_chunks; cc += 64)
+          L = fmaf(wsh[ncp + cc * G + p], exp2f(wsh[cc * G + p] - mx), L);
+        const float invL = 1.f / wave_sum(L);
+        for (int cc = lane; cc < n_chunks; cc += 64)
+          wsh[cc * G + p] = exp2f(wsh[cc * G + p] - mx) * invL;
+      }
+      __syncthreads();
+      for (int it = tid; it < G * kD; it += kThreads) {
+        const int p = it / kD;
+        const int dim = it - p * kD;
+        const float* po = pbase + p * (kD + 2) + dim;
+        float O = 0.f;
+        for (int c0 = 0; c0 < n_chunks; c0 += 32) {
+          float v[32];
+#pragma unroll
+          for (int j = 0; j < 32; ++j) v[j] = c0 + j < n_chunks ? ld_agent(&po[(c0 + j) * cstride]) : 0.f;
+#pragma unroll
+          for (int j = 0; j < 32; ++j)
+            if (c0 + j < n_chunks) O = fmaf(v[j], wsh[(c0 + j) * G + p], O);
+        }
+        store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim, O);
+      }
+    } else {  // more chunks than the LDS weights hold: two passes per output
+      for (int it = tid; it < G * kD; it += kThreads) {
+        const int p = it / kD;
+        const int dim = it - p * kD;
+        float M = -INFINITY;
+#pragma unroll 8
+        for (int cc = 0; cc < n_chunks; ++cc)
+          M = fmaxf(M, ld_agent(&pbase[cc * cstride + p * (kD + 2) + kD]));
+        float L = 0.f, O = 0.f;
+#pragma unroll 8
+        for (int cc = 0; cc < n_chunks; ++cc) {
+          const float* pc = pbase + cc * cstride + p * (kD + 2);
+          const float f = exp2f(ld_agent(&pc[kD]) - M);
+          L = fmaf(ld_agent(&pc[kD + 1]), f, L);
+          O = fmaf(ld_agent(&pc[dim]), f, O);
+        }
+        store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G + p) * kD + dim,
+                  O / L);
+      }
     }
-  }
-  if (tid == 0) __hip_atomic_store(&a.ws_cnt[r * g.H + h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0)
+      __hip_atomic_store(&a.ws_cnt[r * g.H + h], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
 
   // One segment: the tiles [t0, t1) of request r (its chunk c of n_chunks) for head h. IN_RANGE: one
   // of several that its workgroup walks.
   auto segment = [&](const Segment& q, bool& need_luts, const auto& a, Smem& S, uint16_t* lut3s,
                      int tid, auto in_range) __attribute__((always_inline)) {
-  constexpr bool IN_RANGE = decltype(in_range)::value;
-  // (a copy: through a generic reference its fields would be loaded from memory in every tile)
-  const Geom g = a.g;
-  const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
-  if (IN_RANGE && tid == 0) S.sg = q;  // read back behind the barriers below
-  const int h = q.h, r = q.r, c = q.c, seq = q.seq, qrow_r = q.qrow, dslot = q.dslot, t0 = q.t0,
-            t1 = q.t1;
-  // What the tile loop takes of the arguments. A chunk's go through opaque copies: the compiler would
-  // otherwise load some of them from the argument segment again in every tile, and each such load
-  // waits for the LDS reads in flight. (A range's tile loop was 5 % slower with the copies.)
-  const uint8_t* page = a.page;
-  const float* cs_cache = a.cs_cache;
-  int64_t n_slots = a.n_slots, slot_stride = a.slot_stride;
-  int block_size = a.block_size, bs_shift = a.bs_shift;
-  float scale_log2 = a.scale_log2;
-  if constexpr (!IN_RANGE)
-    __asm__("" : "+s"(page), "+s"(cs_cache), "+s"(n_slots), "+s"(slot_stride), "+s"(block_size),
-                 "+s"(bs_shift), "+s"(scale_log2));
-  const int ptok = tid >> 2;  // token / part handled by this thread in prefetch + commit
-  const int part = tid & 3;
-  // block id of this thread's token in the first tile (position clamped into the context)
-  const int64_t bt_row = (int64_t)r * a.bt_row_stride;
-  const int pos0 = min(t0 + ptok, seq - 1);
-  const int bi0 = bs_shift >= 0 ? pos0 >> bs_shift : pos0 / block_size;
-  const int64_t qrow = qrow_r;
-  const int blk_t0 = seq > 0 ? a.bt[bt_row + bi0] : -1;
-  if (seq <= 0) {  // empty context: the reference's einsum over zero rows is 0
-    for (int i = tid; i < G * kD; i += kThreads)
-      store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G) * kD + i, 0.f);
-    return;
-  }
-  // This chunk's block ids (at most kSegMax, host-bounded), requested in the same round trip as
-  // the first tile's block id and the decoder slot: they depend on the plan only, and are staged
-  // into LDS after the code tables are built.
-  const int bfirst = t0 / block_size;
-  const int nseg = (t1 - 1) / block_size - bfirst + 1;
-  constexpr int kSegPer = (kSegMax + kThreads - 1) / kThreads;
-  int segv[kSegPer];
-#pragma unroll
-  for (int k = 0; k < kSegPer; ++k) {
-    const int i = tid + kThreads * k;
-    segv[k] = i < nseg ? a.bt[bt_row + bfirst + i] : -1;
-  }
-
-  // The first tile's bytes (bad block ids are flagged when the chunk's ids are staged); the
-  // decoder slot (the device registry keyed by the request's first block) came with the plan
-  const int k_row_off = g.k_field + h * g.k_row;
-  const int v_row_off = g.k_slot + h * g.v_row;
-  // the rows' 64-byte windows (16-aligned; each row lies inside its window, host-checked)
-  const int k_win = k_row_off & ~15, v_win = v_row_off & ~15;
-  RawSlotW<KU, CM> P;
-  {
-    const uint8_t* base = nullptr;
-    if (ptok < min(kTile, t1 - t0) && blk_t0 >= 0 && blk_t0 < a.num_blocks) {
-      const int64_t slot = (int64_t)blk_t0 * block_size + (pos0 - bi0 * block_size);
-      if (slot < n_slots) base = page + slot * slot_stride;
-    }
-    fetch_raw_slot_w<KU, CM>(P, base, part, g, k_win, v_win);
-  }
-  if (dslot < 0 || dslot >= a.n_dec_slots) {
-    if (tid == 0) atomicOr(a.err, TTKV_ERR_NO_DECODER);
-    if (c == 0)
+    constexpr bool IN_RANGE = decltype(in_range)::value;
+    // (a copy: through a generic reference its fields would be loaded from memory in every tile)
+    const Geom g = a.g;
+    const int lane = tid & 63, wv = tid >> 6, n = lane & 15, gq = lane >> 4;
+    if (IN_RANGE && tid == 0) S.sg = q;  // read back behind the barriers below
+    const int h = q.h, r = q.r, c = q.c, seq = q.seq, qrow_r = q.qrow, dslot = q.dslot, t0 = q.t0,
+              t1 = q.t1;
+    // What the tile loop takes of the arguments. A chunk's go through opaque copies: the compiler would
+    // otherwise load some of them from the argument segment again in every tile, and each such load
+    // waits for the LDS reads in flight. (A range's tile loop was 5 % slower with the copies.)
+    const uint8_t* page = a.page;
+    const float* cs_cache = a.cs_cache;
+    int64_t n_slots = a.n_slots, slot_stride = a.slot_stride;
+    int block_size = a.block_size, bs_shift = a.bs_shift;
+    float scale_log2 = a.scale_log2;
+    if constexpr (!IN_RANGE)
+      __asm__("" : "+s"(page), "+s"(cs_cache), "+s"(n_slots), "+s"(slot_stride), "+s"(block_size),
+                   "+s"(bs_shift), "+s"(scale_log2));
+    const int ptok = tid >> 2;  // token / part handled by this thread in prefetch + commit
+    const int part = tid & 3;
+    // block id of this thread's token in the first tile (position clamped into the context)
+    const int64_t bt_row = (int64_t)r * a.bt_row_stride;
+    const int pos0 = min(t0 + ptok, seq - 1);
+    const int bi0 = bs_shift >= 0 ? pos0 >> bs_shift : pos0 / block_size;
+    const int64_t qrow = qrow_r;
+    const int blk_t0 = seq > 0 ? a.bt[bt_row + bi0] : -1;
+    if (seq <= 0) {  // empty context: the reference's einsum over zero rows is 0
       for (int i = tid; i < G * kD; i += kThreads)
-        store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G) * kD + i, NAN);
-    return;
-  }
-
-  // ---- decoder and query values for the MFMA fragments: loaded now, so that their latency
-  // overlaps the table and block-id staging
-  const int dl = 16 * wv + 4 * gq;
-  const int HD = g.H * kD;
-  // int8 ranks 32s + 8gq .. +7 of each of the lane's two columns (one 8-byte load per step; the
-  // k = 16 tail step: ranks 32 KSTEPS + 4gq .. +3, 4 bytes) and their rulers (one float4 per 4
-  // ranks, the same for both columns). 16 KU <= R, so every load is inside the decoder.
-  const int R = dec_ranks(g.r1);
-  const int8_t* decq = a.dec_q + ((int64_t)dslot * HD + h * kD) * R;
-  const float* decs = a.dec_scale + (int64_t)dslot * R;
-  u32x2v dq[2][KSTEPS];
-  uint32_t dqt[2] = {0u, 0u};
-  float4v dsc[2 * KSTEPS + 1];
-#pragma unroll
-  for (int mi = 0; mi < 2; ++mi) {
-    const int8_t* col = decq + (int64_t)(16 * (wv + 4 * mi) + n) * R;
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) dq[mi][s] = *gbl((const u32x2v*)(col + 32 * s + 8 * gq));
-    if constexpr (KTAIL) dqt[mi] = *gbl((const uint32_t*)(col + 32 * KSTEPS + 4 * gq));
-  }
-#pragma unroll
-  for (int s = 0; s < KSTEPS; ++s) {
-    dsc[2 * s] = *gbl((const float4v*)(decs + 32 * s + 8 * gq));
-    dsc[2 * s + 1] = *gbl((const float4v*)(decs + 32 * s + 8 * gq + 4));
-  }
-  dsc[2 * KSTEPS] = KTAIL ? *gbl((const float4v*)(decs + 32 * KSTEPS + 4 * gq))
-                          : float4v{0.f, 0.f, 0.f, 0.f};
-  // (rows n >= G of the fragment are zero: they load head G - 1 and discard it, so the loads
-  // carry no branch and go out together)
-  float qraw[8];
-  {
-    const bool qvec = act_rows_aligned(a.q, a.q_dtype, a.q_row_stride);
-    const int64_t qb = qrow * a.q_row_stride + (int64_t)(h * G + min(n, G - 1)) * kD;
-    load_act_n<4>(a.q, a.q_dtype, qb + dl, qvec, qraw);
-    load_act_n<4>(a.q, a.q_dtype, qb + 64 + dl, qvec, qraw + 4);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qraw[j] = n < G ? qraw[j] : 0.f;
-  }
-
-  // ---- code tables, and this chunk's block ids
-  if (need_luts) build_luts(S.lut, (RB == 3 || VB == 3) ? lut3s : nullptr, tid, kThreads);
-  need_luts = false;  // (a segment without tokens or decoder returns before this)
-#pragma unroll
-  for (int k = 0; k < kSegPer; ++k) {
-    const int i = tid + kThreads * k;
-    if (i < nseg) {
-      int blk = segv[k];
-      if (blk < 0 || blk >= a.num_blocks) {
-        atomicOr(a.err, TTKV_ERR_BAD_BLOCK);
-        blk = -1;
-      }
-      S.seg[i] = blk;
+        store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G) * kD + i, 0.f);
+      return;
     }
-  }
-
-  // slot bases are 16-aligned, so a row's byte misalignment is fixed per head
-  const uint32_t ksel = stage_selector(k_row_off & 3, part != 0);
-  const uint32_t vsel = stage_selector(v_row_off & 3, part != 0);
-  // fp8 code unit of the hardware conversion (2^-9 for OCP e4m3, 2^-10 for FNUZ); codes of 4
-  // bits are converted as plain bytes
-  const float inv_unit = 1.0f / __builtin_amdgcn_cvt_pk_f32_fp8(1, false)[0];
-  const float inv_unit_k = RB == 3 ? inv_unit : 1.0f;
-
-  __syncthreads();  // seg
-
-  auto slot_base = [&](int tt) -> const uint8_t* {
-    if (ptok >= min(kTile, t1 - tt)) return nullptr;
-    const int pos = tt + ptok;
-    const int bi = bs_shift >= 0 ? pos >> bs_shift : pos / block_size;
-    const int blk = S.seg[bi - bfirst];
-    if (blk < 0) return nullptr;
-    const int64_t slot = (int64_t)blk * block_size + (pos - bi * block_size);
-    if (slot >= n_slots) return nullptr;
-    return page + slot * slot_stride;
-  };
-
-  // ---- decoder fragments (A operand, M = dims, K = r1), hi/lo fp16, resident in registers.
-  half8 ahi[2][KSTEPS], alo[2][KSTEPS];
-  half8 thi[2], tlo[2];  // k = 16 tail step (odd KU), upper halves zero
+    // This chunk's block ids (at most kSegMax, host-bounded), requested in the same round trip as
+    // the first tile's block id and the decoder slot: they depend on the plan only, and are staged
+    // into LDS after the code tables are built.
+    const int bfirst = t0 / block_size;
+    const int nseg = (t1 - 1) / block_size - bfirst + 1;
+    constexpr int kSegPer = (kSegMax + kThreads - 1) / kThreads;
+    int segv[kSegPer];
 #pragma unroll
-  for (int mi = 0; mi < 2; ++mi) {
+    for (int k = 0; k < kSegPer; ++k) {
+      const int i = tid + kThreads * k;
+      segv[k] = i < nseg ? a.bt[bt_row + bfirst + i] : -1;
+    }
+
+    // The first tile's bytes (bad block ids are flagged when the chunk's ids are staged); the
+    // decoder slot (the device registry keyed by the request's first block) came with the plan
+    const int k_row_off = g.k_field + h * g.k_row;
+    const int v_row_off = g.k_slot + h * g.v_row;
+    // the rows' 64-byte windows (16-aligned; each row lies inside its window, host-checked)
+    const int k_win = k_row_off & ~15, v_win = v_row_off & ~15;
+    RawSlotW<KU, CM> P;
+    {
+      const uint8_t* base = nullptr;
+      if (ptok < min(kTile, t1 - t0) && blk_t0 >= 0 && blk_t0 < a.num_blocks) {
+        const int64_t slot = (int64_t)blk_t0 * block_size + (pos0 - bi0 * block_size);
+        if (slot < n_slots) base = page + slot * slot_stride;
+      }
+      fetch_raw_slot_w<KU, CM>(P, base, part, g, k_win, v_win);
+    }
+    if (dslot < 0 || dslot >= a.n_dec_slots) {
+      if (tid == 0) atomicOr(a.err, TTKV_ERR_NO_DECODER);
+      if (c == 0)
+        for (int i = tid; i < G * kD; i += kThreads)
+          store_act(a.out, a.out_dtype, qrow * a.out_row_stride + (int64_t)(h * G) * kD + i, NAN);
+      return;
+    }
+
+    // ---- decoder and query values for the MFMA fragments: loaded now, so that their latency
+    // overlaps the table and block-id staging
+    const int dl = 16 * wv + 4 * gq;
+    const int HD = g.H * kD;
+    // int8 ranks 32s + 8gq .. +7 of each of the lane's two columns (one 8-byte load per step; the
+    // k = 16 tail step: ranks 32 KSTEPS + 4gq .. +3, 4 bytes) and their rulers (one float4 per 4
+    // ranks, the same for both columns). 16 KU <= R, so every load is inside the decoder.
+    const int R = dec_ranks(g.r1);
+    const int8_t* decq = a.dec_q + ((int64_t)dslot * HD + h * kD) * R;
+    const float* decs = a.dec_scale + (int64_t)dslot * R;
+    u32x2v dq[2][KSTEPS];
+    uint32_t dqt[2] = {0u, 0u};
+    float4v dsc[2 * KSTEPS + 1];
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) {
+      const int8_t* col = decq + (int64_t)(16 * (wv + 4 * mi) + n) * R;
+#pragma unroll
+      for (int s = 0; s < KSTEPS; ++s) dq[mi][s] = *gbl((const u32x2v*)(col + 32 * s + 8 * gq));
+      if constexpr (KTAIL) dqt[mi] = *gbl((const uint32_t*)(col + 32 * KSTEPS + 4 * gq));
+    }
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
-      float v[8];
-      dec_values4(dq[mi][s][0], dsc[2 * s], v);
-      dec_values4(dq[mi][s][1], dsc[2 * s + 1], v + 4);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float f = 32 * s + 8 * gq + j < g.r1 ? v[j] : 0.f;
-        const _Float16 hi = (_Float16)f;
-        ahi[mi][s][j] = hi;
-        alo[mi][s][j] = (_Float16)(f - (float)hi);
-      }
+      dsc[2 * s] = *gbl((const float4v*)(decs + 32 * s + 8 * gq));
+      dsc[2 * s + 1] = *gbl((const float4v*)(decs + 32 * s + 8 * gq + 4));
     }
-    float vt[4];
-    dec_values4(dqt[mi], dsc[2 * KSTEPS], vt);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float f = KTAIL && j < 4 && 32 * KSTEPS + 4 * gq + j < g.r1 ? vt[j & 3] : 0.f;
-      const _Float16 hi = (_Float16)f;
-      thi[mi][j] = hi;
-      tlo[mi][j] = (_Float16)(f - (float)hi);
-    }
-  }
-
-  // ---- query fragments (A operand of q.k, M = heads, K = this wave's 32 dims in the order of
-  // the rotated-key fragments: 8*gq + i <-> dim dl + i, 8*gq + 4 + i <-> dim 64 + dl + i),
-  // split hi + lo in fp16; rows >= G are zero.
-  half8 qhi, qlo;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const _Float16 hi = (_Float16)qraw[j];
-    qhi[j] = hi;
-    qlo[j] = (_Float16)(qraw[j] - (float)hi);
-  }
-
-  // P.V accumulators on MFMA: O^T[dims, heads] for the wave's two dim tiles; lane (n, gq) holds
-  // dims 4gq..4gq+3 of the tile for query head n (n < G; the other columns stay zero)
-  float4v oacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  float m_run[G], l_lane[G];
-#pragma unroll
-  for (int p = 0; p < G; ++p) {
-    m_run[p] = -INFINITY;
-    l_lane[p] = 0.f;
-  }
-  // P' = P * ruler_v is carried at scale 2^-ve so that it stays an fp16 normal below 2^15: P <=
-  // 2^8 (lazy rescale), so every ruler of a tile must stay below 2^(7 + ve). ve starts at 0 (no
-  // scaling: rulers below 128, i.e. V rows up to |v| ~ 384 at 3 bits) and grows, behind a ballot,
-  // when a tile brings a larger ruler; the accumulators are then rescaled by an exact power of
-  // two, and the output takes 2^ve back at the end. Every wave sees the same rulers, so ve is
-  // the same in all of them.
-  int ve = 0;
-  float v_thr = 128.f, v_mul = 1.f;
-  // V^T A-fragments come from the decoded code rows through the LDS transpose read: in each
-  // 16-lane group, lanes 2j and 2j+1 address the two 8-byte halves of row j (token 8gq + j) of
-  // the tile's 16 dims, and lane n receives column n (dim n) of those 8 rows, i.e. exactly
-  // A[dim n][tokens 8gq .. 8gq+7].
-  const int tr_tok = 8 * gq + (n >> 1);
-  const int tr_col = 8 * (n & 1);
-
-  // RoPE angle rows (shared by every request and head, L2-resident): this lane's 4 dims of the
-  // token it reconstructs in block nb, requested one block ahead inside the reconstruction. Block
-  // 0's row of the NEXT tile is requested after the reconstruction, where the registers allow.
-  constexpr bool kAngle0Ahead = G <= 4;
-  float4v cv0, sv0;
-  auto angle_row = [&](int ts, int nb, float4v& cv, float4v& sv) {
-    const int tok = 16 * nb + n;
-    const uint32_t pos = tok < min(kTile, t1 - ts) ? ts + tok : ts;  // (a sign would be extended)
-    cv = *gbl((const float4v*)&cs_cache[(int64_t)pos * kD + dl]);
-    sv = *gbl((const float4v*)&cs_cache[(int64_t)pos * kD + 64 + dl]);
-  };
-  if constexpr (kAngle0Ahead) angle_row(t0, 0, cv0, sv0);
-
-  for (int tt = t0, tp = 0; tt < t1; tt += kTile, tp ^= 1) {
-    const int ntile = min(kTile, t1 - tt);
-    // the next tile's slot address first: its block-id read overlaps the commit
-    const uint8_t* next_base = tt + kTile < t1 ? slot_base(tt + kTile) : nullptr;
-    // ---------------------------------------------------------------- commit prefetched bytes
+    dsc[2 * KSTEPS] = KTAIL ? *gbl((const float4v*)(decs + 32 * KSTEPS + 4 * gq))
+                            : float4v{0.f, 0.f, 0.f, 0.f};
+    // (rows n >= G of the fragment are zero: they load head G - 1 and discard it, so the loads
+    // carry no branch and go out together)
+    float qraw[8];
     {
-      const float cs = commit_coef<KU, CM>(P, (uint32_t*)&S.coef[ptok][0], part, g);
-      if (part == 0) S.cs[ptok] = cs;
-      stage_row_w(P.krow, (k_row_off & 15) >> 2, ksel, &S.rawk[ptok][part * 4]);
-      stage_row_w(P.vrow, (v_row_off & 15) >> 2, vsel, &S.rawv[ptok][part * 4]);
+      const bool qvec = act_rows_aligned(a.q, a.q_dtype, a.q_row_stride);
+      const int64_t qb = qrow * a.q_row_stride + (int64_t)(h * G + min(n, G - 1)) * kD;
+      load_act_n<4>(a.q, a.q_dtype, qb + dl, qvec, qraw);
+      load_act_n<4>(a.q, a.q_dtype, qb + 64 + dl, qvec, qraw + 4);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) qraw[j] = n < G ? qraw[j] : 0.f;
     }
-    // No barrier: wave w commits and decodes the same 16 tokens (16w .. 16w+15), and LDS
-    // accesses of one wave complete in order (the fences only keep the compiler from moving
-    // them). The buffers this tile writes are free: the previous tile's reconstruction read
-    // coef / kcode / kr before the last barrier, and its softmax and P.V read the other parity of
-    // vcode / vr / f.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // The next tile's slot bytes, requested as soon as the commit has freed P: they arrive during
-    // the decode and reconstruction instead of stalling the next commit (measured: the bytes took
-    // ~2k cycles, longer than the softmax and P.V they used to overlap). The reconstruction's
-    // angle loads queue behind them (loads complete in order) but are issued a decode later.
-    if (tt + kTile < t1) fetch_raw_slot_w<KU, CM>(P, next_base, part, g, k_win, v_win);
-    // ---------------------------------------------------------------- decode (thread = half row)
-    // The decode and reconstruction are each workgroup's critical chain; the co-resident
-    // workgroup's softmax, P.V and commit fill the issue slots they leave. Raising this wave's
-    // priority for these two phases lets them run ahead (headline 172 -> 159 us, measured).
-    __builtin_amdgcn_s_setprio(1);
-    {
-      // lanes 0..31: K rows, 32..63: V rows of this wave's 16 tokens, two threads per row; one
-      // decode call with per-lane row and destination (the two kinds share the code width)
-      const bool is_v = lane >= 32;
-      const int tok = 16 * wv + ((lane >> 1) & 15);
-      const int half = lane & 1;
-      const uint32_t* row = is_v ? S.rawv[tok] : S.rawk[tok];
-      uint8_t* dst = is_v ? &S.vcode[tp][tok][64 * half] : &S.kcode[tok][64 * half];
-      decode_half_row_be<RB>(row, half, S.lut, lut3s, dst);
-      if (half == 0) {
-        const float rul = f16_bits_to_float(staged_u16(row, kBitmapBytes + (is_v ? g.v_pb : g.k_pb)));
-        if (is_v) {
-          S.vr[tp][tok] = rul;
-        } else {
-          const float cs = S.cs[tok];
-          // the hardware reciprocal (1 ulp) instead of an IEEE divide, which would lengthen the
-          // K lanes' branch
-          S.kr[tok] = cs != 0.f ? rul * inv_unit_k * __builtin_amdgcn_rcpf(cs) : 0.f;
-          S.f[tp][tok] = cs * scale_log2;
+
+    // ---- code tables, and this chunk's block ids
+    if (need_luts) build_luts(S.lut, (RB == 3 || VB == 3) ? lut3s : nullptr, tid, kThreads);
+    need_luts = false;  // (a segment without tokens or decoder returns before this)
+#pragma unroll
+    for (int k = 0; k < kSegPer; ++k) {
+      const int i = tid + kThreads * k;
+      if (i < nseg) {
+        int blk = segv[k];
+        if (blk < 0 || blk >= a.num_blocks) {
+          atomicOr(a.err, TTKV_ERR_BAD_BLOCK);
+          blk = -1;
         }
+        S.seg[i] = blk;
       }
     }
-    __syncthreads();
-    // ---------------------------------------------------------------- recon + rope + q.k
-    float4v cvn, svn;
-    if constexpr (kAngle0Ahead) {
-      cvn = cv0;
-      svn = sv0;
-    } else {
-      angle_row(tt, 0, cvn, svn);
-    }
-    // Software-pipelined over the 4 token blocks: block nb + 1's MFMAs are issued before block nb's
-    // epilogue (residual, RoPE, hi/lo split, scores), which has no dependence on them, so the two
-    // overlap within the wave (reconstruction phase 3.65k -> 3.17k cycles per tile, measured).
-    auto recon_mfma = [&](int nb, float krp, float4v& acc0, float4v& acc1) {
-      const int tok = 16 * nb + n;
-      // 4-bit codes arrive as c: the -8 * ruler offset enters as the accumulator's start
-      const float kb = RB == 4 ? -8.f * krp : 0.f;
-      acc0 = float4v{kb, kb, kb, kb};
-      acc1 = float4v{kb, kb, kb, kb};
+
+    // slot bases are 16-aligned, so a row's byte misalignment is fixed per head
+    const uint32_t ksel = stage_selector(k_row_off & 3, part != 0);
+    const uint32_t vsel = stage_selector(v_row_off & 3, part != 0);
+    // fp8 code unit of the hardware conversion (2^-9 for OCP e4m3, 2^-10 for FNUZ); codes of 4
+    // bits are converted as plain bytes
+    const float inv_unit = 1.0f / __builtin_amdgcn_cvt_pk_f32_fp8(1, false)[0];
+    const float inv_unit_k = RB == 3 ? inv_unit : 1.0f;
+
+    __syncthreads();  // seg
+
+    auto slot_base = [&](int tt) -> const uint8_t* {
+      if (ptok >= min(kTile, t1 - tt)) return nullptr;
+      const int pos = tt + ptok;
+      const int bi = bs_shift >= 0 ? pos >> bs_shift : pos / block_size;
+      const int blk = S.seg[bi - bfirst];
+      if (blk < 0) return nullptr;
+      const int64_t slot = (int64_t)blk * block_size + (pos - bi * block_size);
+      if (slot >= n_slots) return nullptr;
+      return page + slot * slot_stride;
+    };
+
+    // ---- decoder fragments (A operand, M = dims, K = r1), hi/lo fp16, resident in registers.
+    half8 ahi[2][KSTEPS], alo[2][KSTEPS];
+    half8 thi[2], tlo[2];  // k = 16 tail step (odd KU), upper halves zero
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) {
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) {
-        const half8 b = *(const half8*)&S.coef[tok][32 * s + 8 * gq];
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[0][s], b, acc0, 0, 0, 0);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[0][s], b, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[1][s], b, acc1, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[1][s], b, acc1, 0, 0, 0);
-      }
-      if constexpr (KTAIL) {
-        // The k = 16 tail runs as a 16x16x32 step whose upper k half is zero in A and B (lane
-        // (n, gq) holds k 8gq..8gq+7 of a 32-wide step; the tail's k 4gq..4gq+3 sit in its first
-        // four). One MFMA shape per accumulator chain: on gfx950 a 16x16x16 step reading a
-        // 16x16x32 step's result as its accumulator gave wrong sums when the compiler placed the
-        // two a few instructions apart (measured; extra wait states between them also fixed it).
-        const half4 b4 = *(const half4*)&S.coef[tok][32 * KSTEPS + 4 * gq];
-        const half8 b = {b4[0], b4[1], b4[2], b4[3], 0, 0, 0, 0};
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(thi[0], b, acc0, 0, 0, 0);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tlo[0], b, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(thi[1], b, acc1, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tlo[1], b, acc1, 0, 0, 0);
-      }
-    };
-    float krA = S.kr[n];
-    float4v accA0, accA1;
-    recon_mfma(0, krA, accA0, accA1);
+        float v[8];
+        dec_values4(dq[mi][s][0], dsc[2 * s], v);
+        dec_values4(dq[mi][s][1], dsc[2 * s + 1], v + 4);
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int tok = 16 * nb + n;
-      const float4v cv = cvn, sv = svn;
-      if (nb < 3) angle_row(tt, nb + 1, cvn, svn);
-      float4v accB0 = accA0, accB1 = accA1;
-      float krB = krA;
-      if (nb < 3) {
-        krB = S.kr[tok + 16];
-        recon_mfma(nb + 1, krB, accB0, accB1);
-      }
-      float vl[4], vh[4];
-      codes4<RB>(*(const uint32_t*)&S.kcode[tok][dl], vl);
-      codes4<RB>(*(const uint32_t*)&S.kcode[tok][64 + dl], vh);
-      float y[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float kl = fmaf(krA, vl[i], accA0[i]);
-        const float kh = fmaf(krA, vh[i], accA1[i]);
-        y[i] = kl * cv[i] - kh * sv[i];
-        y[4 + i] = kh * cv[i] + kl * sv[i];
-      }
-      half8 yhi, ylo;
-      split8(y, yhi, ylo);
-      float4v sacc = {0.f, 0.f, 0.f, 0.f};
-      sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qhi, yhi, sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qhi, ylo, sacc, 0, 0, 0);
-      if constexpr (QLO) sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qlo, yhi, sacc, 0, 0, 0);
-      // lane (n, gq) holds heads 4*gq .. 4*gq+3 of token n
-      if (4 * gq < G) *(float4v*)&S.spart[wv][tok][4 * gq] = sacc;
-      accA0 = accB0;
-      accA1 = accB1;
-      krA = krB;
-    }
-    __builtin_amdgcn_s_setprio(0);
-    // ---------------------------------------------------------------- next tile's first angle row
-    if constexpr (kAngle0Ahead)
-      if (tt + kTile < t1) angle_row(tt + kTile, 0, cv0, sv0);
-    __syncthreads();
-    // ---------------------------------------------------------------- online softmax (every wave)
-    {
-      const bool valid = lane < ntile;
-      const float ft = S.f[tp][lane];
-      const float vrt = S.vr[tp][lane];
-      float sum[kSP];
-#pragma unroll
-      for (int i = 0; i < kSP; ++i) sum[i] = 0.f;
-#pragma unroll
-      for (int ww = 0; ww < kWaves; ++ww) {
-#pragma unroll
-        for (int i = 0; i < kSP; i += 4) {
-          const float4v x = *(const float4v*)&S.spart[ww][lane][i];
-          sum[i] += x[0];
-          sum[i + 1] += x[1];
-          sum[i + 2] += x[2];
-          sum[i + 3] += x[3];
+        for (int j = 0; j < 8; ++j) {
+          const float f = 32 * s + 8 * gq + j < g.r1 ? v[j] : 0.f;
+          const _Float16 hi = (_Float16)f;
+          ahi[mi][s][j] = hi;
+          alo[mi][s][j] = (_Float16)(f - (float)hi);
         }
       }
-      float amul = 1.f;  // this lane's factor for its head column n of the P.V accumulators
-      if (__builtin_amdgcn_ballot_w64(vrt >= v_thr) != 0) {  // rare: a large V ruler
-        // rulers are >= 0: the biased exponent field orders them; vrt < 2^(ex + 1)
-        const int ex = wave_max_i((int)(__float_as_uint(vrt) >> 23) - 127);
-        const int ve_new = ex - 6;
-        amul = ldexpf(1.f, ve - ve_new);
-        ve = ve_new;
-        v_thr = ldexpf(1.f, 7 + ve);
-        v_mul = ldexpf(1.f, -ve);
-      }
-      const float vrs = vrt * v_mul;
+      float vt[4];
+      dec_values4(dqt[mi], dsc[2 * KSTEPS], vt);
 #pragma unroll
-      for (int p = 0; p < G; ++p) {
-        const float s = valid ? sum[p] * ft : -INFINITY;
-        // Lazy rescaling: the reference point m_run only moves when some score exceeds it by
-        // more than 2^8, so most tiles skip the wave-wide max (p stays <= 256; fp32 has the
-        // range). m_run is the same in every lane and wave (same inputs), so the branch is
-        // uniform.
-        if (__builtin_amdgcn_ballot_w64(s > m_run[p] + 8.f) != 0) {
-          const float mt = wave_max(s);
-          const float alpha = exp2f(m_run[p] - mt);
-          m_run[p] = mt;
-          l_lane[p] *= alpha;
-          amul = n == p ? alpha * amul : amul;
-        }
-        const float pr = fast_exp2(s - m_run[p]);
-        l_lane[p] += pr;
-        // P' = P * ruler_v * 2^-ve, rounded to fp16 once (the V codes are exact integers);
-        // tokens past the tile's end have P = 0 and all-zero decoded rows
-        S.pw[wv][p][lane] = (_Float16)(pr * vrs);
-      }
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi) oacc[mi] *= amul;
-    }
-    // ---------------------------------------------------------------- P.V on MFMA
-    // O^T[dims, heads] += V^T[dims, tokens] * P'^T[tokens, heads], 32 tokens per k-step. The B
-    // operand (lane (n, gq): P' of head n, tokens 8gq..8gq+7) is this wave's own LDS row, written
-    // just above by other lanes of the wave: LDS accesses of one wave complete in order, and the
-    // wavefront fence keeps the compiler from reordering them.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      half8 bp = {};
-      if (n < G) bp = *(const half8*)&S.pw[wv][n][32 * kk + 8 * gq];
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi) {
-        const uint8_t* src = &S.vcode[tp][32 * kk + tr_tok][16 * (wv + 4 * mi) + tr_col];
-        typedef int v2i __attribute__((ext_vector_type(2)));
-        const v2i raw = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-            (__attribute__((address_space(3))) v2i*)(src));
-        half8 av;
-        if constexpr (VB == 3) {
-          // fp8 bytes of (c - 4) scaled by the fp8 unit's inverse: exact small integers
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const half2v lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(raw[w], inv_unit, false);
-            const half2v hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(raw[w], inv_unit, true);
-            av[4 * w] = lo[0];
-            av[4 * w + 1] = lo[1];
-            av[4 * w + 2] = hi[0];
-            av[4 * w + 3] = hi[1];
-          }
-        } else {
-          // offset-binary code bytes c -> fp16 (c - 8), exact: 1024 + c from the byte placed
-          // under the fp16 exponent of 1024, minus 1032
-          const half2v bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, (uint32_t)raw[w], 0x04010400u);
-            const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, (uint32_t)raw[w], 0x04030402u);
-            const half2v a = __builtin_bit_cast(half2v, lo) - bias;
-            const half2v b = __builtin_bit_cast(half2v, hi) - bias;
-            av[4 * w] = a[0];
-            av[4 * w + 1] = a[1];
-            av[4 * w + 2] = b[0];
-            av[4 * w + 3] = b[1];
-          }
-        }
-        oacc[mi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bp, oacc[mi], 0, 0, 0);
+      for (int j = 0; j < 8; ++j) {
+        const float f = KTAIL && j < 4 && 32 * KSTEPS + 4 * gq + j < g.r1 ? vt[j & 3] : 0.f;
+        const _Float16 hi = (_Float16)f;
+        thi[mi][j] = hi;
+        tlo[mi][j] = (_Float16)(f - (float)hi);
       }
     }
-  }
 
-  if constexpr (IN_RANGE) {
-    // What the rest needs of the segment and of the arguments is read again here, so that it does
-    // not take registers through the tile loop.
-    const DecodeArgs AS4* end = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();
-    __asm__ volatile("" : "+s"(end));
-    auto rfl = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
-    finish(*end, S, tid, rfl(S.sg.h), rfl(S.sg.r), rfl(S.sg.c), rfl(S.sg.n_chunks), rfl(S.sg.base),
-           rfl(S.sg.qrow), oacc, m_run, l_lane, ve);
-  } else {
-    finish(a, S, tid, h, r, c, q.n_chunks, q.base, qrow, oacc, m_run, l_lane, ve);
-  }
+    // ---- query fragments (A operand of q.k, M = heads, K = this wave's 32 dims in the order of
+    // the rotated-key fragments: 8*gq + i <-> dim dl + i, 8*gq + 4 + i <-> dim 64 + dl + i),
+    // split hi + lo in fp16; rows >= G are zero.
+    half8 qhi, qlo;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const _Float16 hi = (_Float16)qraw[j];
+      qhi[j] = hi;
+      qlo[j] = (_Float16)(qraw[j] - (float)hi);
+    }
+
+    // P.V accumulators on MFMA: O^T[dims, heads] for the wave's two dim tiles; lane (n, gq) holds
+    // dims 4gq..4gq+3 of the tile for query head n (n < G; the other columns stay zero)
+    float4v oacc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    float m_run[G], l_lane[G];
+#pragma unroll
+    for (int p = 0; p < G; ++p) {
+      m_run[p] = -INFINITY;
+      l_lane[p] = 0.f;
+    }
+    // P' = P * ruler_v is carried at scale 2^-ve so that it stays an fp16 normal below 2^15: P <=
+    // 2^8 (lazy rescale), so every ruler of a tile must stay below 2^(7 + ve). ve starts at 0 (no
+    // scaling: rulers below 128, i.e. V rows up to |v| ~ 384 at 3 bits) and grows, behind a ballot,
+    // when a tile brings a larger ruler; the accumulators are then rescaled by an exact power of
+    // two, and the output takes 2^ve back at the end. Every wave sees the same rulers, so ve is
+    // the same in all of them.
+    int ve = 0;
+    float v_thr = 128.f, v_mul = 1.f;
+    // V^T A-fragments come from the decoded code rows through the LDS transpose read: in each
+    // 16-lane group, lanes 2j and 2j+1 address the two 8-byte halves of row j (token 8gq + j) of
+    // the tile's 16 dims, and lane n receives column n (dim n) of those 8 rows, i.e. exactly
+    // A[dim n][tokens 8gq .. 8gq+7].
+    const int tr_tok = 8 * gq + (n >> 1);
+    const int tr_col = 8 * (n & 1);
+
+    // RoPE angle rows (shared by every request and head, L2-resident): this lane's 4 dims of the
+    // token it reconstructs in block nb, requested one block ahead inside the reconstruction. Block
+    // 0's row of the NEXT tile is requested after the reconstruction, where the registers allow.
+    constexpr bool kAngle0Ahead = G <= 4;
+    float4v cv0, sv0;
+    auto angle_row = [&](int ts, int nb, float4v& cv, float4v& sv) {
+      const int tok = 16 * nb + n;
+      const uint32_t pos = tok < min(kTile, t1 - ts) ? ts + tok : ts;  // (a sign would be extended)
+      cv = *gbl((const float4v*)&cs_cache[(int64_t)pos * kD + dl]);
+      sv = *gbl((const float4v*)&cs_cache[(int64_t)pos * kD + 64 + dl]);
+    };
+    if constexpr (kAngle0Ahead) angle_row(t0, 0, cv0, sv0);
+
+    for (int tt = t0, tp = 0; tt < t1; tt += kTile, tp ^= 1) {
+      const int ntile = min(kTile, t1 - tt);
+      // the next tile's slot address first: its block-id read overlaps the commit
+      const uint8_t* next_base = tt + kTile < t1 ? slot_base(tt + kTile) : nullptr;
+      // ---------------------------------------------------------------- commit prefetched bytes
+      {
+        const float cs = commit_coef<KU, CM>(P, (uint32_t*)&S.coef[ptok][0], part, g);
+        if (part == 0) S.cs[ptok] = cs;
+        stage_row_w(P.krow, (k_row_off & 15) >> 2, ksel, &S.rawk[ptok][part * 4]);
+        stage_row_w(P.vrow, (v_row_off & 15) >> 2, vsel, &S.rawv[ptok][part * 4]);
+      }
+      // No barrier: wave w commits and decodes the same 16 tokens (16w .. 16w+15), and LDS
+      // accesses of one wave complete in order (the fences only keep the compiler from moving
+      // them). The buffers this tile writes are free: the previous tile's reconstruction read
+      // coef / kcode / kr before the last barrier, and its softmax and P.V read the other parity of
+      // vcode / vr / f.
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // The next tile's slot bytes, requested as soon as the commit has freed P: they arrive during
+      // the decode and reconstruction instead of stalling the next commit (measured: the bytes took
+      // ~2k cycles, longer than the softmax and P.V they used to overlap). The reconstruction's
+      // angle loads queue behind them (loads complete in order) but are issued a decode later.
+      if (tt + kTile < t1) fetch_raw_slot_w<KU, CM>(P, next_base, part, g, k_win, v_win);
+      // ---------------------------------------------------------------- decode (thread = half row)
+      // The decode and reconstruction are each workgroup's critical chain; the co-resident
+      // workgroup's softmax, P.V and commit fill the issue slots they leave. Raising this wave's
+      // priority for these two phases lets them run ahead (headline 172 -> 159 us, measured).
+      __builtin_amdgcn_s_setprio(1);
+      {
+        // lanes 0..31: K rows, 32..63: V rows of this wave's 16 tokens, two threads per row; one
+        // decode call with per-lane row and destination (the two kinds share the code width)
+        const bool is_v = lane >= 32;
+        const int tok = 16 * wv + ((lane >> 1) & 15);
+        const int half = lane & 1;
+        const uint32_t* row = is_v ? S.rawv[tok] : S.rawk[tok];
+        uint8_t* dst = is_v ? &S.vcode[tp][tok][64 * half] : &S.kcode[tok][64 * half];
+        decode_half_row_be<RB>(row, half, S.lut, lut3s, dst);
+        if (half == 0) {
+          const float rul = f16_bits_to_float(staged_u16(row, kBitmapBytes + (is_v ? g.v_pb : g.k_pb)));
+          if (is_v) {
+            S.vr[tp][tok] = rul;
+          } else {
+            const float cs = S.cs[tok];
+            // the hardware reciprocal (1 ulp) instead of an IEEE divide, which would lengthen the
+            // K lanes' branch
+            S.kr[tok] = cs != 0.f ? rul * inv_unit_k * __builtin_amdgcn_rcpf(cs) : 0.f;
+            S.f[tp][tok] = cs * scale_log2;
+          }
+        }
+      }
+      __syncthreads();
+      // ---------------------------------------------------------------- recon + rope + q.k
+      float4v cvn, svn;
+      if constexpr (kAngle0Ahead) {
+        cvn = cv0;
+        svn = sv0;
+      } else {
+        angle_row(tt, 0, cvn, svn);
+      }
+      // Software-pipelined over the 4 token blocks: block nb + 1's MFMAs are issued before block nb's
+      // epilogue (residual, RoPE, hi/lo split, scores), which has no dependence on them, so the two
+      // overlap within the wave (reconstruction phase 3.65k -> 3.17k cycles per tile, measured).
+      auto recon_mfma = [&](int nb, float krp, float4v& acc0, float4v& acc1) {
+        const int tok = 16 * nb + n;
+        // 4-bit codes arrive as c: the -8 * ruler offset enters as the accumulator's start
+        const float kb = RB == 4 ? -8.f * krp : 0.f;
+        acc0 = float4v{kb, kb, kb, kb};
+        acc1 = float4v{kb, kb, kb, kb};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+          const half8 b = *(const half8*)&S.coef[tok][32 * s + 8 * gq];
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[0][s], b, acc0, 0, 0, 0);
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[0][s], b, acc0, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[1][s], b, acc1, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[1][s], b, acc1, 0, 0, 0);
+        }
+        if constexpr (KTAIL) {
+          // The k = 16 tail runs as a 16x16x32 step whose upper k half is zero in A and B (lane
+          // (n, gq) holds k 8gq..8gq+7 of a 32-wide step; the tail's k 4gq..4gq+3 sit in its first
+          // four). One MFMA shape per accumulator chain: on gfx950 a 16x16x16 step reading a
+          // 16x16x32 step's result as its accumulator gave wrong sums when the compiler placed the
+          // two a few instructions apart (measured; extra wait states between them also fixed it).
+          const half4 b4 = *(const half4*)&S.coef[tok][32 * KSTEPS + 4 * gq];
+          const half8 b = {b4[0], b4[1], b4[2], b4[3], 0, 0, 0, 0};
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(thi[0], b, acc0, 0, 0, 0);
+          acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tlo[0], b, acc0, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(thi[1], b, acc1, 0, 0, 0);
+          acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(tlo[1], b, acc1, 0, 0, 0);
+        }
+      };
+      float krA = S.kr[n];
+      float4v accA0, accA1;
+      recon_mfma(0, krA, accA0, accA1);
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        const int tok = 16 * nb + n;
+        const float4v cv = cvn, sv = svn;
+        if (nb < 3) angle_row(tt, nb + 1, cvn, svn);
+        float4v accB0 = accA0, accB1 = accA1;
+        float krB = krA;
+        if (nb < 3) {
+          krB = S.kr[tok + 16];
+          recon_mfma(nb + 1, krB, accB0, accB1);
+        }
+        float vl[4], vh[4];
+        codes4<RB>(*(const uint32_t*)&S.kcode[tok][dl], vl);
+        codes4<RB>(*(const uint32_t*)&S.kcode[tok][64 + dl], vh);
+        float y[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float kl = fmaf(krA, vl[i], accA0[i]);
+          const float kh = fmaf(krA, vh[i], accA1[i]);
+          y[i] = kl * cv[i] - kh * sv[i];
+          y[4 + i] = kh * cv[i] + kl * sv[i];
+        }
+        half8 yhi, ylo;
+        split8(y, yhi, ylo);
+        float4v sacc = {0.f, 0.f, 0.f, 0.f};
+        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qhi, yhi, sacc, 0, 0, 0);
+        sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qhi, ylo, sacc, 0, 0, 0);
+        if constexpr (QLO) sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qlo, yhi, sacc, 0, 0, 0);
+        // lane (n, gq) holds heads 4*gq .. 4*gq+3 of token n
+        if (4 * gq < G) *(float4v*)&S.spart[wv][tok][4 * gq] = sacc;
+        accA0 = accB0;
+        accA1 = accB1;
+        krA = krB;
+      }
+      __builtin_amdgcn_s_setprio(0);
+      // ---------------------------------------------------------------- next tile's first angle row
+      if constexpr (kAngle0Ahead)
+        if (tt + kTile < t1) angle_row(tt + kTile, 0, cv0, sv0);
+      __syncthreads();
+      // ---------------------------------------------------------------- online softmax (every wave)
+      {
+        const bool valid = lane < ntile;
+        const float ft = S.f[tp][lane];
+        const float vrt = S.vr[tp][lane];
+        float sum[kSP];
+#pragma unroll
+        for (int i = 0; i < kSP; ++i) sum[i] = 0.f;
+#pragma unroll
+        for (int ww = 0; ww < kWaves; ++ww) {
+#pragma unroll
+          for (int i = 0; i < kSP; i += 4) {
+            const float4v x = *(const float4v*)&S.spart[ww][lane][i];
+            sum[i] += x[0];
+            sum[i + 1] += x[1];
+            sum[i + 2] += x[2];
+            sum[i + 3] += x[3];
+          }
+        }
+        float amul = 1.f;  // this lane's factor for its head column n of the P.V accumulators
+        if (__builtin_amdgcn_ballot_w64(vrt >= v_thr) != 0) {  // rare: a large V ruler
+          // rulers are >= 0: the biased exponent field orders them; vrt < 2^(ex + 1)
+          const int ex = wave_max_i((int)(__float_as_uint(vrt) >> 23) - 127);
+          const int ve_new = ex - 6;
+          amul = ldexpf(1.f, ve - ve_new);
+          ve = ve_new;
+          v_thr = ldexpf(1.f, 7 + ve);
+          v_mul = ldexpf(1.f, -ve);
+        }
+        const float vrs = vrt * v_mul;
+#pragma unroll
+        for (int p = 0; p < G; ++p) {
+          const float s = valid ? sum[p] * ft : -INFINITY;
+          // Lazy rescaling: the reference point m_run only moves when some score exceeds it by
+          // more than 2^8, so most tiles skip the wave-wide max (p stays <= 256; fp32 has the
+          // range). m_run is the same in every lane and wave (same inputs), so the branch is
+          // uniform.
+          if (__builtin_amdgcn_ballot_w64(s > m_run[p] + 8.f) != 0) {
+            const float mt = wave_max(s);
+            const float alpha = exp2f(m_run[p] - mt);
+            m_run[p] = mt;
+            l_lane[p] *= alpha;
+            amul = n == p ? alpha * amul : amul;
+          }
+          const float pr = fast_exp2(s - m_run[p]);
+          l_lane[p] += pr;
+          // P' = P * ruler_v * 2^-ve, rounded to fp16 once (the V codes are exact integers);
+          // tokens past the tile's end have P = 0 and all-zero decoded rows
+          S.pw[wv][p][lane] = (_Float16)(pr * vrs);
+        }
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) oacc[mi] *= amul;
+      }
+      // ---------------------------------------------------------------- P.V on MFMA
+      // O^T[dims, heads] += V^T[dims, tokens] * P'^T[tokens, heads], 32 tokens per k-step. The B
+      // operand (lane (n, gq): P' of head n, tokens 8gq..8gq+7) is this wave's own LDS row, written
+      // just above by other lanes of the wave: LDS accesses of one wave complete in order, and the
+      // wavefront fence keeps the compiler from reordering them.
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        half8 bp = {};
+        if (n < G) bp = *(const half8*)&S.pw[wv][n][32 * kk + 8 * gq];
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) {
+          const uint8_t* src = &S.vcode[tp][32 * kk + tr_tok][16 * (wv + 4 * mi) + tr_col];
+          typedef int v2i __attribute__((ext_vector_type(2)));
+          const v2i raw = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+              (__attribute__((address_space(3))) v2i*)(src));
+          half8 av;
+          if constexpr (VB == 3) {
+            // fp8 bytes of (c - 4) scaled by the fp8 unit's inverse: exact small integers
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+              const half2v lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(raw[w], inv_unit, false);
+              const half2v hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(raw[w], inv_unit, true);
+              av[4 * w] = lo[0];
+              av[4 * w + 1] = lo[1];
+              av[4 * w + 2] = hi[0];
+              av[4 * w + 3] = hi[1];
+            }
+          } else {
+            // offset-binary code bytes c -> fp16 (c - 8), exact: 1024 + c from the byte placed
+            // under the fp16 exponent of 1024, minus 1032
+            const half2v bias = {(_Float16)1032.0f, (_Float16)1032.0f};
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+              const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, (uint32_t)raw[w], 0x04010400u);
+              const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, (uint32_t)raw[w], 0x04030402u);
+              const half2v a = __builtin_bit_cast(half2v, lo) - bias;
+              const half2v b = __builtin_bit_cast(half2v, hi) - bias;
+              av[4 * w] = a[0];
+              av[4 * w + 1] = a[1];
+              av[4 * w + 2] = b[0];
+              av[4 * w + 3] = b[1];
+            }
+          }
+          oacc[mi] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bp, oacc[mi], 0, 0, 0);
+        }
+      }
+    }
+
+    if constexpr (IN_RANGE) {
+      // What the rest needs of the segment and of the arguments is read again here, so that it does
+      // not take registers through the tile loop.
+      const DecodeArgs AS4* end = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();
+      __asm__ volatile("" : "+s"(end));
+      auto rfl = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+      finish(*end, S, tid, rfl(S.sg.h), rfl(S.sg.r), rfl(S.sg.c), rfl(S.sg.n_chunks), rfl(S.sg.base),
+             rfl(S.sg.qrow), oacc, m_run, l_lane, ve);
+    } else {
+      finish(a, S, tid, h, r, c, q.n_chunks, q.base, qrow, oacc, m_run, l_lane, ve);
+    }
   };
 
   // A chunk's segment has a body of its own, without the loop and what it needs: with one body for
@@ -1198,10 +1203,10 @@ struct DecodeShape {
   int64_t items_cap;  // (request, chunk, head) items any batch of this shape can need
 };
 
-// The kernel picks its chunk length from the batch's token total T: 64 * ceil(T * H / target / 64),
-// clamped to [64, chunk_cap]. The batch with every request at max_seq_len gives the longest
-// chunk and bounds the item count when the cap binds; otherwise the items are at most
-// sum_r (seq_r / chunk + 1) * H <= target + num_reqs * H.
+// The kernel takes the shortest chunk whose items fit whole rounds of `target`, at most chunk_cap.
+// The batch with every request at max_seq_len gives the longest chunk and bounds the item count
+// when the cap binds; otherwise the items are at most target + num_reqs * H. A range plan has at
+// most target / H teams, and at most (teams + num_reqs) * H partials.
 static DecodeShape decode_shape(int num_reqs, int H, int max_seq_len, int block_size) {
   DecodeShape s;
   s.target = 2 * device_cu_count();  // one round at 2 resident blocks per CU
