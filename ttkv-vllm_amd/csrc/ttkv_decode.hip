@@ -632,17 +632,12 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
     if (IN_RANGE && tid == 0) S.sg = q;  // read back behind the barriers below
     const int h = q.h, r = q.r, c = q.c, seq = q.seq, qrow_r = q.qrow, dslot = q.dslot, t0 = q.t0,
               t1 = q.t1;
-    // What the tile loop takes of the arguments. A chunk's go through opaque copies: the compiler would
-    // otherwise load some of them from the argument segment again in every tile, and each such load
-    // waits for the LDS reads in flight. (A range's tile loop was 5 % slower with the copies.)
+    // what the tile loop takes of the arguments
     const uint8_t* page = a.page;
     const float* cs_cache = a.cs_cache;
-    int64_t n_slots = a.n_slots, slot_stride = a.slot_stride;
-    int block_size = a.block_size, bs_shift = a.bs_shift;
-    float scale_log2 = a.scale_log2;
-    if constexpr (!IN_RANGE)
-      __asm__("" : "+s"(page), "+s"(cs_cache), "+s"(n_slots), "+s"(slot_stride), "+s"(block_size),
-                   "+s"(bs_shift), "+s"(scale_log2));
+    const int64_t n_slots = a.n_slots, slot_stride = a.slot_stride;
+    const int block_size = a.block_size, bs_shift = a.bs_shift;
+    const float scale_log2 = a.scale_log2;
     const int ptok = tid >> 2;  // token / part handled by this thread in prefetch + commit
     const int part = tid & 3;
     // block id of this thread's token in the first tile (position clamped into the context)
@@ -1095,12 +1090,16 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
 
   // A chunk's segment has a body of its own, without the loop and what it needs: with one body for
   // both, batches of like lengths took 2 to 8 % longer than without ranges (8 x 14,402: 125.1 us against
-  // 120.5, 64 x 1,182 .. 1,712: 117.5 against 108.4), with two 120.3 and 107.2. It is said to be the
-  // likely one so that its blocks stay together (1 x 4,000: 28.2 us against 28.7). S and lut3s are
-  // parameters of both lambdas so that each body folds their addresses into its LDS offsets.
+  // 120.5, 64 x 1,182 .. 1,712: 117.5 against 108.4), with two 120.4 and 107.7. What keeps the two bodies
+  // apart: the arguments read through an opaque pointer (loaded once for both ahead of the plan, they
+  // do not fit the scalar registers: 4-bit coefficients, 8 x 14,402: 121.6 us against 119), S and
+  // lut3s as parameters (each body folds their addresses into its LDS offsets), and the hint that
+  // this one is likely (its blocks stay together: 1 x 4,000 28.0 us against 28.6).
   bool need_luts = true;
   if (__builtin_expect(!ranges, 1)) {
-    segment(q, need_luts, a, S, lut3s, (int)threadIdx.x, std::false_type{});
+    const DecodeArgs AS4* ap = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();
+    __asm__("" : "+s"(ap));
+    segment(q, need_luts, *ap, S, lut3s, (int)threadIdx.x, std::false_type{});
     return;
   }
   for (;;) {
