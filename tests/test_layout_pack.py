@@ -3,7 +3,9 @@ slot bytes the REFERENCE wrote (tests/golden/ref_encode_*.npz: `fit_k_slots`, `f
 `v_slots`, with the coefficients and rulers they were packed from), against the oracle's packer
 on random row stores, and by round trips. Reference: vllm_ttkv/layout.py:161-261 and its test
 tests/test_layout.py (pack, then unpack, must be a faithful rearrangement)."""
+import collections
 import copy
+import dataclasses
 import pathlib
 import pickle
 from types import SimpleNamespace
@@ -101,3 +103,16 @@ def test_copies_hold_the_fields_alone():
     for twin in (pickle.loads(fresh), copy.copy(lay), copy.deepcopy(lay)):
         assert twin == lay and "_c_struct" not in twin.__dict__
         assert twin.compressed_bytes_per_token() == lay.compressed_bytes_per_token()
+
+
+def test_c_struct_of_a_layout_without_a_dict():
+    """Any object with a layout's fields has a C struct; one that cannot keep it gets a new one."""
+    lay = play.layout_for_config(play.CONFIGS["safe"], 110)
+    names = [f.name for f in dataclasses.fields(lay)]
+    for twin in (collections.namedtuple("L", names)(*(getattr(lay, n) for n in names)),
+                 dataclasses.make_dataclass("S", names, frozen=True, slots=True)(
+                     *(getattr(lay, n) for n in names)),
+                 SimpleNamespace(**{n: getattr(lay, n) for n in names})):
+        assert bytes(_hip.Layout.of(twin)) == bytes(_hip.Layout.of(lay))
+    twin.H = 4                                # (the namespace's fields can change)
+    assert _hip.Layout.of(twin).H == 4

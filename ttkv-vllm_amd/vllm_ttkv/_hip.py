@@ -32,15 +32,16 @@ class Layout(ctypes.Structure):
 
     @classmethod
     def of(cls, lay) -> "Layout":
-        """The C struct of a layout, kept with it (its fields are frozen, and the library only
+        """The C struct of a layout, kept with it where its fields are frozen (the library only
         reads the struct)."""
-        c = lay.__dict__.get("_c_struct")
+        kept = getattr(lay, "__dict__", {})
+        c = kept.get("_c_struct")
         if c is None:
             c = cls(lay.H, lay.d, lay.r1, lay.qbits, lay.res_k, lay.res_bits, lay.v_lanes,
                     lay.v_bits)
-            if getattr(type(lay), "__dataclass_params__", None) is not None \
-                    and type(lay).__dataclass_params__.frozen:
-                lay.__dict__["_c_struct"] = c
+            params = getattr(type(lay), "__dataclass_params__", None)
+            if params is not None and params.frozen:
+                kept["_c_struct"] = c
         return c
 
 
