@@ -270,6 +270,14 @@ struct TileTokens {
 __device__ TileTokens find_tile(const WriteArgs& a, int tile) {
   const int lane = threadIdx.x & 63;
   const int s0 = a.tok0, s1 = a.tok0 + a.num_tokens;
+  if (a.num_reqs == 1) {  // by scalar arithmetic (the scan costs 1 us of 47 with 2,048 tokens)
+    const int q0 = min(max(a.qsl[0], s0), s1), q1 = min(max(a.qsl[1], q0), s1);
+    const int head = (q0 - s0 + kTok - 1) / kTok, mid = (q1 - q0 + kTok - 1) / kTok;
+    const bool in_head = tile < head, in_mid = !in_head && tile < head + mid;
+    const int lo = in_head ? s0 : in_mid ? q0 : q1, hi = in_head ? q0 : in_mid ? q1 : s1;
+    const int first = lo + (tile - (in_head ? 0 : in_mid ? head : head + mid)) * kTok;
+    return {first - s0, min(kTok, max(hi - first, 0)), in_mid ? a.bt[0] : -1};
+  }
   int before = 0;
   for (int j0 = 0; j0 < a.num_reqs + 2; j0 += 64) {  // span j: request j - 1
     const int j = j0 + lane, r = j - 1;
