@@ -208,9 +208,10 @@ int64_t ttkv_prefill_workspace_bytes(const ttkv_layout* lay, int32_t num_heads, 
  * Chunks of two or more queries (G <= 4, r1 <= 128) run as two launches: every stored key is
  * decoded and reconstructed once into the workspace (rotated key hi + lo fp16, exact V codes, V
  * rulers), then flash attention on MFMA reads it for every 128-query block (96 at G = 4). Single
- * queries (and G = 8 or r1 > 128; G = 4 with a workspace too small for the tiles) run one fused launch
- * that reconstructs each key tile once per 64-query block. Scores never leave the chip. Precision as for ttkv_decode_paged (the softmax weight times
- * the V ruler rounded to fp16 once, at a power-of-two scale that keeps it below 2^15).
+ * queries (and r1 > 128; G = 4 with a workspace too small for the tiles) run one fused launch that
+ * reconstructs each key tile once per 64-query block. G > 4 is refused. Scores never leave the
+ * chip. Precision as for ttkv_decode_paged (the softmax weight times the V ruler rounded to fp16
+ * once, at a power-of-two scale that keeps it below 2^15).
  * req_index    optional [num_reqs] int32: batch rows to process (block_table / seq_lens /
  *              query_start_loc are indexed by it); NULL = rows 0..num_reqs-1.
  * max_q_len / max_seq_len bound Q and n over the processed rows (they size the grid).

@@ -1095,11 +1095,12 @@ __global__ __launch_bounds__(kThreads, 2) void decode_paged_kernel(DecodeArgs a)
 
   // A chunk's segment has a body of its own, without the loop and what it needs: with one body for
   // both, batches of like lengths took 2 to 8 % longer than without ranges (8 x 14,402: 125.1 us against
-  // 120.5, 64 x 1,182 .. 1,712: 117.5 against 108.4), with two 120.4 and 107.7. What keeps the two bodies
-  // apart: the arguments read through an opaque pointer (loaded once for both ahead of the plan, they
-  // do not fit the scalar registers: 4-bit coefficients, 8 x 14,402: 121.6 us against 119), S and
-  // lut3s as parameters (each body folds their addresses into its LDS offsets), and the hint that
-  // this one is likely (its blocks stay together: 1 x 4,000 28.0 us against 28.6).
+  // 120.5, 64 x 1,182 .. 1,712: 117.5 against 108.4), with two 120.4 and 107.7; ranges take about 1 %
+  // longer with two (64 x 40 .. 1,700: 84.7 us against 82.8). What keeps the two bodies apart: the
+  // arguments read through an opaque pointer (loaded once for both ahead of the plan, they do not
+  // fit the scalar registers: 4-bit coefficients, 8 x 14,402: 121.6 us against 119), S and lut3s as
+  // parameters (each body folds their addresses into its LDS offsets), and the hint that this one
+  // is likely (its blocks stay together: 1 x 4,000 28.0 us against 28.6).
   bool need_luts = true;
   if (__builtin_expect(!ranges, 1)) {
     const DecodeArgs AS4* ap = (const DecodeArgs AS4*)__builtin_amdgcn_kernarg_segment_ptr();

@@ -891,7 +891,7 @@ static void launch_project_tiles(const WriteArgs& b, int grid, hipStream_t st) {
 
 // Fewest tokens of a launch that go in tiles: kMinTiled, and kTiledPerReq more for every further
 // request (each can leave a tile partly filled, down to one token). Single tokens against tiles, graph
-// replays, us: one request of 192 tokens 21.4 / 21.8, of 208 22.3 / 21.8, of 1,024 73.8 / 29.3; 2 x 97
+// replays, us: one request of 208 tokens 21.1 / 19.7, of 256 23.1 / 19.8, of 1,024 70.2 / 27.7; 2 x 97
 // 21.2 / 21.1, 8 x 64 42.3 / 21.4, 64 x 4 30.0 / 26.6, 128 x 3 44.6 / 41.5, 256 x 3 83.2 / 76.7, 256 x 2
 // 64.1 / 73.9; one token each of 31 requests and 200 of another 25.1 / 26.6, of 255 and 465 78.2 / 81.4.
 constexpr int kMinTiled = 208, kTiledPerReq = 3;
